@@ -46,8 +46,8 @@ KERNEL_OF_STAGE = {
     "findk0_peak": "simr::k_cc_prep + 2D FFT + simr::k_argmax_*",
     "filter": "simr::k_filter<...> (every band of the stack)",
     "asm_z": "simr::k_asm_z_pair<{zdim}, true> + simr::k_asm_z_pair<{zdim}, false>",
-    "asm_y": "simr::k_asm_y<{ydim}>",
-    "asm_x": "simr::k_asm_x<{xdim}>",
+    "asm_y": "simr::k_asm_y<{ydim}, ...>",
+    "asm_x": "simr::k_asm_phasors + simr::k_asm_x<{xdim}, ...>",
 }
 
 

@@ -230,6 +230,15 @@ Engine::Engine(const simr_params& p, const float* otf, int device) : P(p), L(Lay
   // zoomed assembly lengths), so that no launch path allocates one
   for (int n : {L.nx, L.ny, L.nz, L.xdim, L.ydim, L.zdim})
     if (n > 1) (void)twiddles(n);
+  {
+    AsmParams a{};
+    a.nx = L.nx;
+    a.ny = L.ny;
+    a.xdim = L.xdim;
+    a.ydim = L.ydim;
+    asm_y_request_tables(a);
+    asm_x_request_tables(a);
+  }
   arena_.reserve(L.bytes_total);
   raw_ = arena_.take((size_t)L.nimg * L.nxy_raw * 4);
   bg_ = (float*)arena_.take((size_t)L.nxy_raw * 4);

@@ -286,88 +286,6 @@ __device__ __forceinline__ void fft2_twiddle_all(float2* v, const Fft2Tw<N>& tw)
 // must call it.  WAVE = true: the caller guarantees that the TPT threads of
 // each transform lie in one wavefront and that no other wavefront touches
 // buf during the call; the exchanges then synchronise the wave only.
-// The same with the twiddles read from the table at use (no twiddle
-// registers held across the call; for kernels short of registers).  The
-// scheduling fence after each product stops the compiler from hoisting all
-// N1 loads ahead of the multiplies, which would double the register
-// footprint.
-template <int N, bool INV, bool WAVE = false>
-__device__ __forceinline__ void fft2_lds(float2* buf, int t, const float2* __restrict__ tab) {
-#pragma clang fp contract(off)
-  constexpr F2Plan P = fft2_plan(N);
-  constexpr int N1 = P.n1, N2 = P.n2, MC = N2 / N1, RP = N2 + 1;
-  static_assert(N1 > 0, "no two-pass plan for this length");
-  float2 v[N2];
-  const float2* col = buf + t;
-#pragma unroll
-  for (int c = 0; c < MC; ++c)
-#pragma unroll
-    for (int n1 = 0; n1 < N1; ++n1) v[c * N1 + n1] = col[N2 * n1 + N1 * c];
-  fft2_sync<WAVE>();
-  float2* tcol = buf + t;
-#pragma unroll
-  for (int c = 0; c < MC; ++c) {
-    const int n2 = t + N1 * c;
-    reg_dft<N1, INV>(v + c * N1);
-#pragma unroll
-    for (int k1 = 1; k1 < N1; ++k1) {
-      float2 w = tab[n2 * k1];  // n2 k1 < N2 N1 = N
-      if (INV) w.y = -w.y;
-      v[c * N1 + k1] = cmul(v[c * N1 + k1], w);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) tcol[RP * k1 + N1 * c] = v[c * N1 + k1];
-  }
-  fft2_sync<WAVE>();
-  const float2* row = buf + RP * t;
-#pragma unroll
-  for (int n2 = 0; n2 < N2; ++n2) v[n2] = row[n2];
-  fft2_sync<WAVE>();
-  reg_dft<N2, INV>(v);
-  float2* out = buf + t;
-#pragma unroll
-  for (int k2 = 0; k2 < N2; ++k2) out[N1 * k2] = v[k2];
-  fft2_sync<WAVE>();
-}
-
-// As fft2_lds with table twiddles, with pass 1's inputs already in the
-// thread's registers, v[c N1 + n1] = x[N2 n1 + N1 c + t] (the row is not read
-// from buf; buf only has to be free for this transform when it is called).
-template <int N, bool INV, bool WAVE = false>
-__device__ __forceinline__ void fft2_lds_from_regs(float2* buf, int t, const float2* __restrict__ tab,
-                                                   float2 (&v)[fft2_plan(N).n2]) {
-#pragma clang fp contract(off)
-  constexpr F2Plan P = fft2_plan(N);
-  constexpr int N1 = P.n1, N2 = P.n2, MC = N2 / N1, RP = N2 + 1;
-  static_assert(N1 > 0, "no two-pass plan for this length");
-  float2* tcol = buf + t;
-#pragma unroll
-  for (int c = 0; c < MC; ++c) {
-    const int n2 = t + N1 * c;
-    reg_dft<N1, INV>(v + c * N1);
-#pragma unroll
-    for (int k1 = 1; k1 < N1; ++k1) {
-      float2 w = tab[n2 * k1];
-      if (INV) w.y = -w.y;
-      v[c * N1 + k1] = cmul(v[c * N1 + k1], w);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) tcol[RP * k1 + N1 * c] = v[c * N1 + k1];
-  }
-  fft2_sync<WAVE>();
-  const float2* row = buf + RP * t;
-#pragma unroll
-  for (int n2 = 0; n2 < N2; ++n2) v[n2] = row[n2];
-  fft2_sync<WAVE>();
-  reg_dft<N2, INV>(v);
-  float2* out = buf + t;
-#pragma unroll
-  for (int k2 = 0; k2 < N2; ++k2) out[N1 * k2] = v[k2];
-  fft2_sync<WAVE>();
-}
-
 template <int N, bool INV, bool WAVE = false>
 __device__ __forceinline__ void fft2_lds(float2* buf, int t, const Fft2Tw<N>& tw) {
 #pragma clang fp contract(off)
@@ -401,64 +319,6 @@ __device__ __forceinline__ void fft2_lds(float2* buf, int t, const Fft2Tw<N>& tw
 #pragma unroll
   for (int k2 = 0; k2 < N2; ++k2) out[N1 * k2] = v[k2];
   fft2_sync<WAVE>();
-}
-
-// Register in, register out: pass 1 from the thread's registers
-// (v[c N1 + n1] = x[N2 n1 + N1 c + t]), register twiddles, the transposed
-// intermediate through buf (fft2_span(N) elements), pass 2 into the
-// registers: v[k2] = X[t + N1 k2].  buf is last read by the row reads, so
-// the caller passes a barrier before writing it again.
-template <int N, bool INV, bool WAVE = false>
-__device__ __forceinline__ void fft2_regs(float2* buf, int t, const Fft2Tw<N>& tw, float2 (&v)[fft2_plan(N).n2]) {
-#pragma clang fp contract(off)
-  constexpr F2Plan P = fft2_plan(N);
-  constexpr int N1 = P.n1, N2 = P.n2, MC = N2 / N1, RP = N2 + 1;
-  static_assert(N1 > 0, "no two-pass plan for this length");
-#pragma unroll
-  for (int c = 0; c < MC; ++c) reg_dft<N1, INV>(v + c * N1);
-  fft2_twiddle_all<N, INV>(v, tw);
-  float2* tcol = buf + t;
-#pragma unroll
-  for (int c = 0; c < MC; ++c)
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) tcol[RP * k1 + N1 * c] = v[c * N1 + k1];
-  fft2_sync<WAVE>();
-  const float2* row = buf + RP * t;
-#pragma unroll
-  for (int n2 = 0; n2 < N2; ++n2) v[n2] = row[n2];
-  reg_dft<N2, INV>(v);
-}
-
-// As fft2_lds with register twiddles, but the result stays in the caller's
-// registers: out[k2] = X[t + N1 k2], k2 < N2 (nothing is written back; buf
-// is free again when it returns).
-template <int N, bool INV, bool WAVE = false>
-__device__ __forceinline__ void fft2_lds_regs(float2* buf, int t, const Fft2Tw<N>& tw,
-                                              float2 (&v)[fft2_plan(N).n2]) {
-#pragma clang fp contract(off)
-  constexpr F2Plan P = fft2_plan(N);
-  constexpr int N1 = P.n1, N2 = P.n2, MC = N2 / N1, RP = N2 + 1;
-  static_assert(N1 > 0, "no two-pass plan for this length");
-  const float2* col = buf + t;
-#pragma unroll
-  for (int c = 0; c < MC; ++c)
-#pragma unroll
-    for (int n1 = 0; n1 < N1; ++n1) v[c * N1 + n1] = col[N2 * n1 + N1 * c];
-  fft2_sync<WAVE>();
-#pragma unroll
-  for (int c = 0; c < MC; ++c) reg_dft<N1, INV>(v + c * N1);
-  fft2_twiddle_all<N, INV>(v, tw);
-  float2* tcol = buf + t;
-#pragma unroll
-  for (int c = 0; c < MC; ++c)
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) tcol[RP * k1 + N1 * c] = v[c * N1 + k1];
-  fft2_sync<WAVE>();
-  const float2* row = buf + RP * t;
-#pragma unroll
-  for (int n2 = 0; n2 < N2; ++n2) v[n2] = row[n2];
-  fft2_sync<WAVE>();
-  reg_dft<N2, INV>(v);
 }
 
 }  // namespace simr

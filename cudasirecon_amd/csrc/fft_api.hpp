@@ -9,7 +9,10 @@ namespace simr {
 // the table (hipMalloc and a blocking copy); contexts request every length
 // they use when they are created, so their launch paths only look tables up.
 const float2* twiddles(int n);
-// The same table computed on the device into caller memory (n float2), on stream s.
+// The pass-1 twiddles of the split N = rows x n2 (fft_rp.hpp), arranged
+// [row][n2]: entry i is exp(-2 pi i (i / n2) (i mod n2) / N).  Kept like twiddles().
+const float2* twiddles_rp(int N, int n2);
+// The same table as twiddles(n) computed on the device into caller memory (n float2), on stream s.
 void twiddles_into(float2* out, int n, hipStream_t s);
 bool fft_size_supported(int n);
 

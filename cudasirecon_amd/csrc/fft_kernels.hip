@@ -37,6 +37,30 @@ const float2* twiddles(int N) {
   return d;
 }
 
+namespace {
+std::map<std::pair<int, std::pair<int, int>>, float2*> g_tw_rp;  // (device, (N, n2)), under g_tw_mu
+}  // namespace
+
+const float2* twiddles_rp(int N, int n2) {
+  int dev = 0;
+  SIMR_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(g_tw_mu);
+  const auto key = std::make_pair(dev, std::make_pair(N, n2));
+  auto it = g_tw_rp.find(key);
+  if (it != g_tw_rp.end()) return it->second;
+  std::vector<float2> h(N > 0 ? N : 1);
+  const long double twopi = 6.283185307179586476925286766559L;
+  for (int i = 0; i < N; ++i) {
+    const long double a = -twopi * (long double)((i / n2) * (i % n2)) / (long double)N;
+    h[i] = make_float2((float)cosl(a), (float)sinl(a));
+  }
+  float2* d = nullptr;
+  SIMR_HIP(hipMalloc(&d, sizeof(float2) * h.size()));
+  SIMR_HIP(hipMemcpy(d, h.data(), sizeof(float2) * h.size(), hipMemcpyHostToDevice));
+  g_tw_rp[key] = d;
+  return d;
+}
+
 // exp(-2 pi i m / n) in double (sincospi: the argument is an exact multiple
 // of pi up to the rounding of 2m/n), rounded to float.
 __global__ __launch_bounds__(256) void k_twiddle_table(float2* __restrict__ out, int n) {

@@ -302,8 +302,6 @@ struct FilterBatch {
   FilterBand b[kMaxDirs * kMaxOrders];
 };
 void launch_filter_batch(const FilterParams& p, const FilterBatch& b, hipStream_t s);
-// Fill n float2 with zero.
-void launch_zero(float2* p, long long n, hipStream_t s);
 
 // ---- assembly ----------------------------------------------------------------
 struct AsmParams {
@@ -324,9 +322,15 @@ struct AsmParams {
   // a margin (0: unknown, nothing is skipped)
   float dkx, dky, rc2_zero;
 };
+// Requests the twiddle tables of the y and x passes (nx, ny, xdim, ydim are
+// read), so that their launches do not allocate.
+void asm_y_request_tables(const AsmParams& p);
+void asm_x_request_tables(const AsmParams& p);
+// bands -> stageZ; columns beyond the filter's support are left unwritten
 void launch_asm_z(const AsmParams& p, hipStream_t s);
+// stageZ -> stageY
 void launch_asm_y(const AsmParams& p, hipStream_t s);
-// all assembly bands of stageY -> out (overwritten)
+// all assembly bands of stageY -> out (overwritten); uses stageZ for the phasor table
 void launch_asm_x(const AsmParams& p, hipStream_t s);
 
 }  // namespace simr

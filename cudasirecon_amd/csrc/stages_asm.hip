@@ -17,8 +17,8 @@
 // The order-0 bands of all directions share one transform (linearity).
 #include "device_math.hpp"
 #include "fft.hpp"
-#include "fft2.hpp"
 #include "fft_api.hpp"
+#include "fft_rp.hpp"
 #include "sizes.hpp"
 #include "stages.hpp"
 
@@ -189,26 +189,10 @@ __global__ __launch_bounds__(asm_zp_threads<B0>()) void k_asm_z_pair(AsmParams p
   const int ycp2 = s == p.ny / 2 ? ycs : ycp;        // s = ny/2 is its own mirror
   {
     // The tile's columns lie at |kx| >= x0 dkx on rows |ky| = s dky: when
-    // even the nearest is beyond the filter's support, every input is zero
-    // and so is every output (written without reading or transforming).
+    // even the nearest is beyond the filter's support, every output is zero,
+    // and the y pass does not read it.
     const float kx = (float)x0 * p.dkx, ky = (float)s * p.dky;
-    if (p.rc2_zero > 0.f && kx * kx + ky * ky > p.rc2_zero) {
-      for (int idx = threadIdx.x; idx < W * N; idx += NT) {
-        const int w = idx % W, zout = idx / W;
-        const int xs = x0 + w;
-        if (xs > xmax) continue;
-        float2* plane = p.stageZ + ((long long)a * N + zout) * p.ny * p.nx;
-        const int xd = xs + p.nx / 2 - 1;
-        plane[(long long)ycs * p.nx + xd] = make_float2(0.f, 0.f);
-        plane[(long long)ycp2 * p.nx + xd] = make_float2(0.f, 0.f);
-        if (xs >= 1 && xs <= xmax - 1) {
-          const int xm = p.nx / 2 - 1 - xs;
-          plane[(long long)ycp2 * p.nx + xm] = make_float2(0.f, 0.f);
-          plane[(long long)ycs * p.nx + xm] = make_float2(0.f, 0.f);
-        }
-      }
-      return;  // uniform over the workgroup
-    }
+    if (p.rc2_zero > 0.f && kx * kx + ky * ky > p.rc2_zero) return;  // uniform over the workgroup
   }
   load_twiddles(twr, twstage, threadIdx.x % TPT, tw, threadIdx.x, blockDim.x);
   const long long dirstride = (long long)p.nbands * p.band_stride;
@@ -299,602 +283,104 @@ __global__ __launch_bounds__(asm_zp_threads<B0>()) void k_asm_z_pair(AsmParams p
 }
 
 // ---- y pass: W adjacent xc columns of plane zout (blockIdx.y) of band a (blockIdx.z)
-// Lengths with a wave-local two-pass plan use that core (natural-order LDS
-// columns, register twiddles); the others the radix-stage core.
-template <int N>
-constexpr bool asm_y_fft2() {
-  return use_fft2<N>() && fft2_tpt(N) >= 4;
-}
-template <int N>
-constexpr int asm_y_tpt() {
-  return asm_y_fft2<N>() ? fft2_tpt(N) : fft_tpt(N);
-}
-template <int N>
-constexpr int asm_y_pitch() {
-  return asm_y_fft2<N>() ? fft2_pitch<N>() : lds_pitch(N);
-}
-template <int N>
-__device__ __forceinline__ int asm_y_pos(int Y) {
-  if constexpr (asm_y_fft2<N>())
-    return Y;
-  else
-    return lds_swz<N>(Y);
-}
-// Two-pass tiles hold at most 80 KB, so that two workgroups share a CU;
-// their row segments (8 columns, 64 bytes) pair up in one L2 through the
-// XCD-contiguous tile order.
-template <int N>
-constexpr int asm_y_w() {
-  if (asm_y_fft2<N>()) {
+// Two-pass register core (fft_rp.hpp): every lane loads its pass-1 inputs
+// straight from global memory, the intermediate goes through LDS, and the
+// outputs leave from registers.  HALVES = 2 (exact 2x zoom): the zero-padded
+// transform of N = 2 ny points as the two ny-point halves.
+// Thread (w, j, h): column xc0 + w, lane j of its transform, half h (plans
+// that split the halves); every row access of a wavefront is a W-column
+// segment.  16 columns (whole 128-byte lines) where the workgroup then has
+// at most 512 threads and 80 KB of LDS, so that two share a CU.
+template <int N, int HALVES>
+struct AsmY {
+  static constexpr int LEN = N / HALVES;
+  using K = Rp<LEN, HALVES>;
+  static constexpr int GROUPS = K::T * (K::SPLIT ? 2 : 1);  // lanes of one column
+  static constexpr int span_of(int w) {                     // floats of one transform's LDS
+    const int want = w < 32 ? 32 / w : 1;                   // columns offset by 32 / w banks: conflict-free
+    return K::SPAN + ((want - K::SPAN % 32) % 32 + 32) % 32;
+  }
+  static constexpr int lds_of(int w) { return w * (K::SPLIT ? 2 : 1) * span_of(w) * 4; }
+  static constexpr int width() {
     int w = 16;
-    while (w > 1 && w * asm_y_pitch<N>() * 8 > 80 * 1024) w /= 2;
-    while (w * asm_y_tpt<N>() < 64) w *= 2;
+    while (w > 4 && (w * GROUPS > 512 || lds_of(w) > 80 * 1024)) w /= 2;
+    while (w * K::T < 64) w *= 2;  // whole wavefronts, each within one half
     return w;
   }
-  constexpr int tpt = fft_tpt(N);
-  int w = 1024 / tpt;
-  if (w > 16) w = 16;
-  while (w > 1 && w * lds_pitch(N) * 8 > 80 * 1024) w /= 2;
-  return w;
-}
+  static constexpr int W = width();
+  static constexpr int VALUES = K::R1 * K::HL * K::N1 > K::N2 ? K::R1 * K::HL * K::N1 : K::N2;
+  // wavefronts per SIMD asked of the register allocator (128 VGPRs each at
+  // four, 168 at three): four where that does not spill.  Split halves and
+  // factors of 5 do (800 rows: 29 registers, 243 us against 142 us at three).
+  static constexpr int WAVES = VALUES <= 32 ? (K::SPLIT || LEN % 5 == 0 ? 3 : 4) : VALUES <= 40 ? 2 : 1;
+  static constexpr int NT = W * GROUPS;
+  static constexpr int LDS = lds_of(W);
+};
 
-// Column pitch of the register-in, register-out tiles (exact 2x zoom): a
-// wavefront holds 8 columns x 8 threads, so the pitch is 2 mod 16 (the 16
-// lanes of a 64-bit LDS access land on distinct bank pairs).
-template <int N>
-constexpr int asm_y_pitch_regs() {
-  return asm_y_fft2<N>() ? fft2_span(N) + (18 - fft2_span(N) % 16) % 16 : 1;
-}
-
-// Exact 2x zoom (ny = N/2): slot c N1 + n1 of thread t holds row
-// Y = N2 n1 + N1 c + t of the zero-padded column (source row Y + N/4 - 1 for
-// Y <= N/4, Y - 3N/4 - 1 for Y >= 3N/4 + 1, zero between), read from scol
-// (the column's first element, row stride nx).  The cases are compile-time
-// after unrolling except for a slot that straddles an edge of the zero band.
-template <int N>
-__device__ __forceinline__ void asm_y_fetch_col(const float2* scol, int nx, int ny, float2 (&v)[fft2_plan(N).n2],
-                                                int t) {
-  constexpr int N1 = fft2_plan(N).n1, N2 = fft2_plan(N).n2, MC = N2 / N1;
-  constexpr int H = N / 4, YHI = N - H + 1;
-#pragma unroll
-  for (int c = 0; c < MC; ++c)
-#pragma unroll
-    for (int n1 = 0; n1 < N1; ++n1) {
-      const int Y0 = N2 * n1 + N1 * c;
-      float2& d = v[c * N1 + n1];
-      if (Y0 + N1 - 1 <= H) {
-        d = scol[(long long)(Y0 + t + H - 1) * nx];
-      } else if (Y0 >= YHI) {
-        d = scol[(long long)(Y0 + t - YHI) * nx];
-      } else if (Y0 > H && Y0 + N1 - 1 < YHI) {
-        d = make_float2(0.f, 0.f);
-      } else {
-        const int Y = Y0 + t;
-        const bool lo = Y <= H, hi = Y >= YHI;
-        int sr = lo ? Y + H - 1 : Y - YHI;
-        sr = sr < 0 ? 0 : (sr > ny - 1 ? ny - 1 : sr);
-        const float2 w = scol[(long long)sr * nx];
-        d = (lo || hi) ? w : make_float2(0.f, 0.f);
-      }
-    }
-}
-
-template <int N>
-__global__ __launch_bounds__(asm_y_w<N>() * asm_y_tpt<N>()) void k_asm_y(AsmParams p, const float2* __restrict__ tw) {
-  constexpr bool F2 = asm_y_fft2<N>();
-  constexpr int TPT = asm_y_tpt<N>();
-  constexpr int W = asm_y_w<N>();
-  constexpr int NT = W * TPT;
-  constexpr int LP = asm_y_pitch<N>();
-  static_assert(!F2 || NT % 64 == 0, "two-pass tiles are whole wavefronts");
-  constexpr int LPR = asm_y_pitch_regs<N>();
-  constexpr int LDSN = W * (LP > LPR ? LP : LPR);
-  static_assert(NT <= 1024 && (LDSN + ((N > 1 && !F2) ? N : 1)) * 8 <= 160 * 1024, "the tile fits a workgroup");
-  __shared__ float2 lds[LDSN];
-  FftTw<F2 ? 1 : N> twr;
-  __shared__ float2 twstage[(N > 1 && !F2) ? N : 1];
-  Fft2Tw<F2 ? N : 64> tw2;
-  const bool zoom2 = F2 && 2 * p.ny == N;
-  if constexpr (F2)
-    tw2.load(zoom2 ? threadIdx.x / W : threadIdx.x % TPT, tw);
-  else
-    load_twiddles(twr, twstage, threadIdx.x % TPT, tw, threadIdx.x, blockDim.x);
+template <int N, int HALVES>
+__global__ __launch_bounds__((AsmY<N, HALVES>::NT), (AsmY<N, HALVES>::WAVES)) void k_asm_y(AsmParams p, const float2* __restrict__ tw) {
+  using C = AsmY<N, HALVES>;
+  using K = typename C::K;
+  constexpr int W = C::W, LEN = C::LEN, N1 = K::N1, N2 = K::N2;
+  static_assert(C::NT <= 1024 && C::LDS <= 160 * 1024, "the tile fits a workgroup");
+  __shared__ float buf[C::LDS / 4];
   unsigned bx, by, bz;
   xcd_tile3(bx, by, bz);
   const int a = (int)bz, zout = (int)by;
   const int xc0 = (int)bx * W;
+  float2* const dst = p.stageY + ((long long)a * p.zdim + zout) * (long long)N * p.nx;
   {
     // the tile's column nearest to the centre decides: the dead columns lie
     // at both ends of the row (uniform over the workgroup)
     const int c = p.nx / 2 - 1 < xc0 ? xc0 : (p.nx / 2 - 1 > xc0 + W - 1 ? xc0 + W - 1 : p.nx / 2 - 1);
     if (asm_col_dead(p, c)) {
-      float2* dst = p.stageY + ((long long)a * p.zdim + zout) * (long long)N * p.nx;
-      for (int idx = threadIdx.x; idx < N * W; idx += NT) {
+      for (int idx = threadIdx.x; idx < N * W; idx += C::NT) {
         const int Y = idx / W, w = idx - (idx / W) * W;
         if (xc0 + w < p.nx) dst[(long long)Y * p.nx + xc0 + w] = make_float2(0.f, 0.f);
       }
       return;
     }
   }
-  const float2* src = p.stageZ + ((long long)a * p.zdim + zout) * p.ny * p.nx;
-  if constexpr (F2) {
-    if (zoom2) {
-      // thread (t, w) = (threadIdx.x / W, threadIdx.x % W): column xc0 + w,
-      // pass-1 inputs from global memory into registers, outputs from
-      // registers to global memory; each wavefront's loads and stores cover
-      // whole W-column row segments of 8 consecutive rows, as the staged
-      // copies do, and the padded column never passes through LDS
-      constexpr int N1 = fft2_plan(N).n1, N2 = fft2_plan(N).n2;
-      const int w = threadIdx.x % W, t = threadIdx.x / W;
-      const int xc = xc0 + w < p.nx ? xc0 + w : p.nx - 1;
-      float2 v[N2];
-      asm_y_fetch_col<N>(src + xc, p.nx, p.ny, v, t);
-      fft2_regs<N, true, false>(lds + w * LPR, t, tw2, v);
-      if (xc0 + w < p.nx) {
-        float2* dcol = p.stageY + ((long long)a * p.zdim + zout) * (long long)N * p.nx + xc0 + w;
-#pragma unroll
-        for (int k2 = 0; k2 < N2; ++k2) dcol[(long long)(t + N1 * k2) * p.nx] = v[k2];
-      }
-      return;
-    }
-  }
-  // Source row sr goes to Y = sr - hy (sr >= hy) or Y = sr + N - hy (sr < hy);
-  // the rows between are zero.  Loads run over source rows in batches of B
-  // per thread with clamped addresses and no branches, so a batch is in
-  // flight at once (one batch for a 2x zoom).
+  const int w = threadIdx.x % W, g = threadIdx.x / W;
+  const int j = K::SPLIT ? g % K::T : g;
+  const bool odd = K::SPLIT && g >= K::T;
+  const int xc = xc0 + w < p.nx ? xc0 + w : p.nx - 1;
+  const float2* const src = p.stageZ + ((long long)a * p.zdim + zout) * p.ny * p.nx + xc;
+  // Rows beyond the filter's support in this column are zero; the z pass
+  // does not write them.  The bound is taken a little inside the z pass's
+  // (rc2_zero), so rounding never reads an element that was not written.
+  const float kx = (float)(xc - (p.nx / 2 - 1)) * p.dkx;
+  const float ymax2 = p.rc2_zero > 0.f ? (p.rc2_zero * 0.9999f - kx * kx) : 3.4e38f;
   const int hy = p.ny / 2 - 1;
-  constexpr int B = (N / 2 * W + NT - 1) / NT;
-  const int cnt = p.ny * W;
-  for (int i0 = threadIdx.x; i0 < cnt; i0 += NT * B) {
-    float2 v[B];
+  float2 in[K::R1 * N1];
 #pragma unroll
-    for (int k = 0; k < B; ++k) {
-      const int idx = i0 + k * NT < cnt ? i0 + k * NT : cnt - 1;
-      const int sr = idx / W, w = idx - (idx / W) * W;
-      const int xc = xc0 + w < p.nx ? xc0 + w : p.nx - 1;
-      v[k] = src[(long long)sr * p.nx + xc];
-    }
-#pragma unroll
-    for (int k = 0; k < B; ++k) {
-      const int idx = i0 + k * NT;
-      const int sr = idx / W, w = idx - (idx / W) * W;
-      const int Y = sr >= hy ? sr - hy : sr + N - hy;
-      if (idx < cnt) lds[w * LP + asm_y_pos<N>(Y)] = xc0 + w < p.nx ? v[k] : make_float2(0.f, 0.f);
-    }
-  }
-  for (int idx = threadIdx.x; idx < (N - p.ny) * W; idx += NT) {
-    const int Y = p.ny - p.ny / 2 + 1 + idx / W, w = idx - (idx / W) * W;
-    lds[w * LP + asm_y_pos<N>(Y)] = make_float2(0.f, 0.f);
-  }
-  __syncthreads();
-  if constexpr (F2) {
-    fft2_lds<N, true, true>(lds + (threadIdx.x / TPT) * LP, threadIdx.x % TPT, tw2);
-    __syncthreads();
-  } else {
-    fft_lds<N, true>(lds + (threadIdx.x / TPT) * LP, threadIdx.x % TPT, twr);
-  }
-  float2* dst = p.stageY + ((long long)a * p.zdim + zout) * (long long)N * p.nx;
-  for (int idx = threadIdx.x; idx < N * W; idx += NT) {
-    const int Y = idx / W, w = idx - (idx / W) * W;
-    const int xc = xc0 + w;
-    if (xc < p.nx) dst[(long long)Y * p.nx + xc] = lds[w * LP + asm_y_pos<N>(Y)];
-  }
-}
-
-// ---- x pass: row Y (blockIdx.x) of every output plane.
-// A workgroup transforms G bands of the row at a time (TPT threads each) and
-// walks all bands, so every output element is accumulated in registers and
-// stored once.  The modulation phasors of the row (E per thread for bands
-// 1..kAsmLutBands) are computed once per workgroup and kept in registers for
-// all planes; the FFT twiddles are read from an LDS table.  Lengths with a
-// two-pass plan (N = N1 * N2, fft2.hpp) use that core with G = 8 bands per
-// round (one round for 3 directions x 3 orders); the others use the
-// radix-stage core with 512 threads.
-constexpr int kAsmXBands = 8;
-constexpr int kAsmLutBands = 6;  // 1 + ndirs*(norders-1) <= 7 keeps every phasor in registers
-
-template <int N>
-constexpr bool asm_x_fft2() {
-  return fft2_ok(N) && fft2_tpt(N) >= 8 && 64 % fft2_tpt(N) == 0 && (kAsmXBands * fft2_tpt(N)) % 64 == 0;
-}
-template <int N>
-constexpr int asm_x_tpt() {
-  if (asm_x_fft2<N>()) return fft2_tpt(N);
-  return fft_tpt(N) >= 128 ? 128 : fft_tpt(N);
-}
-// The radix-stage core takes 512 threads (four rows of 128), or 256 (two
-// rows) from 3072-point rows on, so that the rows and the twiddle table fit
-// the 160 KB of LDS.
-template <int N>
-constexpr int asm_x_threads() {
-  return asm_x_fft2<N>() ? kAsmXBands * fft2_tpt(N) : (N >= 3072 ? 256 : 512);
-}
-
-// modulation phasor of assembly band a (>= 1) at output column X of row Y
-// (cos_sin_kernel, gpuFunctionsImpl.cu:1942-1954: float angle, then sin/cos)
-template <int N>
-// 2 (cos, sin) of the modulation phase (the factor 2 of write_outbuffer_kernel2,
-// exact in float, folded in)
-__device__ __forceinline__ float2 asm_phasor(const AsmParams& p, int a, int X, int Y) {
-#pragma clang fp contract(off)
-  const int no = p.norders - 1;
-  const int dir = (a - 1) / no, order = 1 + (a - 1) % no;
-  const float k0x = p.k0[dir].x * (float)order, k0y = p.k0[dir].y * (float)order;
-  const float s1 = (float)(X - N / 2) * k0x;
-  const float s2 = (float)(Y - p.ydim / 2) * k0y;
-  const float sum = s1 + s2;
-  const float angle = (float)((double)p.fact * 3.14159265358979323846 * (double)sum * (double)p.dxyo);
-  float sn, cs;
-  sincosf(angle, &sn, &cs);
-  return make_float2(2.f * cs, 2.f * sn);
-}
-
-// LDS row of one band: natural order for the two-pass core, swizzled for the
-// radix-stage core
-template <int N>
-constexpr int asm_x_pitch() {
-  return asm_x_fft2<N>() ? fft2_span(N) : lds_pitch(N);
-}
-template <int N>
-__device__ __forceinline__ int asm_x_pos(int X) {
-  if constexpr (asm_x_fft2<N>())
-    return X;
-  else
-    return lds_swz<N>(X);
-}
-
-// Adds one transformed band row (band a) in LDS to the row accumulators
-// (write_outbuffer_kernel1/2, gpuFunctionsImpl.cu:1956-1991: band 0 adds its
-// real part, side bands add Re(2 v phasor) with a double intermediate).
-// SRC >= 0: the phasor is lut[.][SRC]; SRC == -1: band 0; SRC == -2: the
-// phasor is computed.  Every table index is a compile-time constant, so the
-// table stays in registers.
-template <int N, int NT, int E, int LB, int SRC>
-__device__ __forceinline__ void asm_x_add_band(const AsmParams& p, const float2* row, int a, int Y,
-                                               float (&acc)[E], const float2 (&lut)[E][LB]) {
-#pragma clang fp contract(off)
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int X = threadIdx.x + e * NT;
-    if (X < N) {
-      const float2 v = row[asm_x_pos<N>(X)];
-      if constexpr (SRC == -1) {
-        acc[e] += v.x;
-      } else {
-        float2 ph;
-        if constexpr (SRC >= 0)
-          ph = lut[e][SRC];
-        else
-          ph = asm_phasor<N>(p, a, X, Y);
-        // 2 v.x cos - 2 v.y sin, ph = 2 (cos, sin): a product and a fused
-        // multiply-add in float.  The reference forms this term in double and
-        // rounds once when adding it to the float output; here the term itself
-        // carries up to an ulp of its larger product, a few 1e-8 of the output,
-        // for a third of the instructions.
-        acc[e] += __builtin_fmaf(v.x, ph.x, -(v.y * ph.y));
-      }
-    }
-  }
-}
-
-// Bands A .. AEND-1 of round R (slot A - R*G), each with its table entry.
-template <int N, int NT, int G, int E, int LB, int R, int A, int AEND>
-__device__ __forceinline__ void asm_x_table_bands(const AsmParams& p, const float2* lds, int Y, float (&acc)[E],
-                                                  const float2 (&lut)[E][LB]) {
-  if constexpr (A < AEND) {
-    constexpr int LP = asm_x_pitch<N>();
-    if (A < p.nasm) {
-      asm_x_add_band<N, NT, E, LB, A == 0 ? -1 : A - 1>(p, lds + (A - R * G) * LP, A, Y, acc, lut);
-      asm_x_table_bands<N, NT, G, E, LB, R, A + 1, AEND>(p, lds, Y, acc, lut);
-    }
-  }
-}
-
-// Adds the G transformed bands of round R (bands R*G + sl in LDS slot sl),
-// in band order.  Band 0 and side bands 1..NTAB come with compile-time table
-// entries (NTAB = LB with the phasor table, 0 without it); the rest compute
-// their phasors.
-template <int N, int NT, int G, int E, int LB, int NTAB, int R>
-__device__ __forceinline__ void asm_x_round(const AsmParams& p, const float2* lds, int a0, int Y, float (&acc)[E],
-                                            const float2 (&lut)[E][LB]) {
-  constexpr int LP = asm_x_pitch<N>();
-  constexpr int A0 = R * G;
-  constexpr int AT = (R < 0) ? 0 : ((A0 + G < NTAB + 1) ? A0 + G : NTAB + 1);  // first band without a table entry
-  int sl = 0;
-  if constexpr (R >= 0 && AT > A0) {
-    asm_x_table_bands<N, NT, G, E, LB, R, A0, AT>(p, lds, Y, acc, lut);
-    sl = AT - A0;
-  }
-  for (; sl < G && a0 + sl < p.nasm; ++sl) asm_x_add_band<N, NT, E, LB, -2>(p, lds + sl * LP, a0 + sl, Y, acc, lut);
-}
-
-// Rows Y of bands a0 .. a0+R-1 of plane zout, each centred in a zero-padded
-// length-N row (ifftshift layout of the zoomed grid), into LDS rows dst,
-// dst + LP, ... by the 64 lanes of one wavefront.  Source column s goes to
-// X = s - (half - 1) for s >= half - 1 and to X = s + N - (half - 1) below;
-// the columns between are zero, and so are bands >= nasm.  The loads run
-// over contiguous source columns in batches of R x B with clamped (always
-// valid) addresses and no branches, so a batch is in flight at once.
-template <int N, int R>
-__device__ __forceinline__ void asm_x_load_rows(const AsmParams& p, float2* dst, int a0, int zout, int Y, int lane) {
-  constexpr int LP = asm_x_pitch<N>();
-  constexpr int B = N >= 256 ? N / 128 : 2;  // one batch for a 2x zoom
-  const int half = p.nx / 2;
-  const float2* src[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int a = a0 + r < p.nasm ? a0 + r : p.nasm - 1;
-    src[r] = p.stageY + (((long long)a * p.zdim + zout) * p.ydim + Y) * p.nx;
-  }
-  for (int s0 = lane; s0 < p.nx; s0 += 64 * B) {
-    float2 v[R][B];
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int k = 0; k < B; ++k) {
-        const int sc = s0 + 64 * k;
-        v[r][k] = src[r][sc < p.nx ? sc : p.nx - 1];
-      }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-      for (int k = 0; k < B; ++k) {
-        const int sc = s0 + 64 * k;
-        const int X = sc >= half - 1 ? sc - (half - 1) : sc + N - (half - 1);
-        if (sc < p.nx) dst[r * LP + asm_x_pos<N>(X)] = a0 + r < p.nasm ? v[r][k] : make_float2(0.f, 0.f);
-      }
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-    for (int X = p.nx - half + 1 + lane; X < N - (half - 1); X += 64) dst[r * LP + asm_x_pos<N>(X)] = make_float2(0.f, 0.f);
-}
-
-// The same rows when the source row fits one batch (nx <= 64 B, every 2x
-// zoom): asm_x_fetch issues the global loads into registers, asm_x_put
-// writes them (and the zero columns) to LDS.  The kernel fetches the next
-// (plane, round) right after putting the current one, so the loads are in
-// flight during the transform and accumulation instead of stalling the
-// start of every plane.
-template <int N>
-constexpr int asm_x_batch() {
-  return N >= 256 ? N / 128 : 2;
-}
-template <int N, int R>
-struct AsmXRows {
-  float2 v[R][asm_x_batch<N>()];
-};
-template <int N, int R>
-__device__ __forceinline__ void asm_x_fetch(const AsmParams& p, AsmXRows<N, R>& b, int a0, int zout, int Y,
-                                            int lane) {
-  constexpr int B = asm_x_batch<N>();
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int a = a0 + r < p.nasm ? a0 + r : p.nasm - 1;
-    const float2* src = p.stageY + (((long long)a * p.zdim + zout) * p.ydim + Y) * p.nx;
-#pragma unroll
-    for (int k = 0; k < B; ++k) {
-      const int sc = lane + 64 * k;
-      b.v[r][k] = src[sc < p.nx ? sc : p.nx - 1];
-    }
-  }
-}
-template <int N, int R>
-__device__ __forceinline__ void asm_x_put(const AsmParams& p, float2* dst, const AsmXRows<N, R>& b, int a0,
-                                          int lane) {
-  constexpr int LP = asm_x_pitch<N>();
-  constexpr int B = asm_x_batch<N>();
-  const int half = p.nx / 2;
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int k = 0; k < B; ++k) {
-      const int sc = lane + 64 * k;
-      const int X = sc >= half - 1 ? sc - (half - 1) : sc + N - (half - 1);
-      if (sc < p.nx) dst[r * LP + asm_x_pos<N>(X)] = a0 + r < p.nasm ? b.v[r][k] : make_float2(0.f, 0.f);
-    }
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-    for (int X = p.nx - half + 1 + lane; X < N - (half - 1); X += 64) dst[r * LP + asm_x_pos<N>(X)] = make_float2(0.f, 0.f);
-}
-
-// Exact 2x zoom (nx = N/2, half = N/4): thread t's pass-1 inputs of row Y
-// of band a, plane zout, loaded straight into registers, slot c N1 + n1
-// holding X = N2 n1 + N1 c + t of the zero-padded row (asm_x_put's layout:
-// X <= N/4 from source column X + N/4 - 1, X >= 3N/4 + 1 from X - 3N/4 - 1,
-// zero between).  The slots' cases are compile-time after unrolling; only a
-// slot that straddles an edge of the zero band tests per thread.
-template <int N>
-__device__ __forceinline__ void asm_x_fetch_cols(const AsmParams& p, float2 (&v)[fft2_plan(N).n2], int a, int zout,
-                                                 int Y, int t) {
-  constexpr int N1 = fft2_plan(N).n1, N2 = fft2_plan(N).n2, MC = N2 / N1;
-  constexpr int H = N / 4, XHI = N - H + 1;
-  const float2* src = p.stageY + (((long long)a * p.zdim + zout) * p.ydim + Y) * p.nx;
-#pragma unroll
-  for (int c = 0; c < MC; ++c)
+  for (int c = 0; c < K::R1; ++c) {
+    const int n2 = K::N2 % K::T == 0 || j + K::T * c < N2 ? j + K::T * c : N2 - 1;
 #pragma unroll
     for (int n1 = 0; n1 < N1; ++n1) {
-      const int X0 = N2 * n1 + N1 * c;
-      float2& d = v[c * N1 + n1];
-      if (X0 + N1 - 1 <= H) {
-        d = src[X0 + t + H - 1];
-      } else if (X0 >= XHI) {
-        d = src[X0 + t - XHI];
-      } else if (X0 > H && X0 + N1 - 1 < XHI) {
-        d = make_float2(0.f, 0.f);
+      const int n = N2 * n1 + n2;
+      // frequency of element n, and its source row (centred: row y + hy)
+      int y;
+      bool live = true;
+      if (HALVES == 2) {
+        y = n > LEN / 2 ? n - LEN : n;
       } else {
-        const int X = X0 + t;
-        const bool lo = X <= H, hi = X >= XHI;
-        int sc = lo ? X + H - 1 : X - XHI;
-        sc = sc < 0 ? 0 : (sc > p.nx - 1 ? p.nx - 1 : sc);
-        const float2 w = src[sc];
-        d = (lo || hi) ? w : make_float2(0.f, 0.f);
+        const bool lo = n <= p.ny - p.ny / 2, hi = n >= N - hy;
+        y = lo ? n : n - N;
+        live = lo || hi;
       }
-    }
-}
-
-template <int N>
-__global__ __launch_bounds__(asm_x_threads<N>(), 2) void k_asm_x(AsmParams p,
-                                                                                   const float2* __restrict__ tw) {
-#pragma clang fp contract(off)
-  constexpr int NT = asm_x_threads<N>();
-  constexpr int TPT = asm_x_tpt<N>();
-  constexpr int G = NT / TPT;
-  constexpr int LP = asm_x_pitch<N>();
-  constexpr int E = (N + NT - 1) / NT;
-  constexpr bool LUT = E <= 4;
-  constexpr int LB = LUT ? kAsmLutBands : 1;
-  static_assert(!asm_x_fft2<N>() || (64 % TPT == 0 && NT % 64 == 0), "two-pass transforms must not straddle waves");
-  static_assert((G * LP + N) * 8 <= 160 * 1024, "band rows and twiddles fit the LDS");
-  __shared__ float2 lds[G * LP];
-  __shared__ float2 twt[N];
-  for (int i = threadIdx.x; i < N; i += NT) twt[i] = tw[i];
-  const int Y = blockIdx.x;
-  const int g = threadIdx.x / TPT, t = threadIdx.x % TPT;
-  const int half = p.nx / 2;
-  float2 lut[E][LB];
-#pragma unroll
-  for (int e = 0; e < E; ++e)
-#pragma unroll
-    for (int b = 0; b < LB; ++b) {
-      const int X = threadIdx.x + e * NT;
-      lut[e][b] = (LUT && X < N && b + 1 < p.nasm) ? asm_phasor<N>(p, b + 1, X, Y) : make_float2(1.f, 0.f);
-    }
-  __syncthreads();
-  if constexpr (asm_x_fft2<N>()) {
-    if (2 * p.nx == N) {
-      // exact 2x zoom: each thread's pass-1 inputs come from global memory
-      // straight into registers (no LDS staging of the padded rows), and the
-      // next (plane, round) is fetched while this one is transformed
-      constexpr int N2 = fft2_plan(N).n2;
-      float2 nxt[N2];
-      asm_x_fetch_cols<N>(p, nxt, g < p.nasm ? g : p.nasm - 1, 0, Y, t);
-      for (int zout = 0; zout < p.zdim; ++zout) {
-        float acc[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) acc[e] = 0.f;
-#pragma nounroll
-        for (int a0 = 0; a0 < p.nasm; a0 += G) {
-          float2 v[N2];
-#pragma unroll
-          for (int i = 0; i < N2; ++i) v[i] = nxt[i];
-          int na0 = a0 + G, nz = zout;
-          if (na0 >= p.nasm) {
-            na0 = 0;
-            ++nz;
-          }
-          if (nz < p.zdim) asm_x_fetch_cols<N>(p, nxt, na0 + g < p.nasm ? na0 + g : p.nasm - 1, nz, Y, t);
-          fft2_lds_from_regs<N, true, true>(lds + g * LP, t, twt, v);
-          __syncthreads();
-          if (a0 == 0)
-            asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, 0>(p, lds, a0, Y, acc, lut);
-          else if (a0 == G)
-            asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, 1>(p, lds, a0, Y, acc, lut);
-          else
-            asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, -1>(p, lds, a0, Y, acc, lut);
-          __syncthreads();
-        }
-        float* orow = p.out + ((long long)zout * p.ydim + Y) * N;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const int X = threadIdx.x + e * NT;
-          if (X < N) orow[X] = acc[e];
-        }
-      }
-      return;
-    }
-    if (p.nx <= 64 * asm_x_batch<N>()) {
-      constexpr int TPW = 64 / TPT;
-      const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-      AsmXRows<N, TPW> rows;
-      asm_x_fetch<N, TPW>(p, rows, wave * TPW, 0, Y, lane);
-      for (int zout = 0; zout < p.zdim; ++zout) {
-        float acc[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) acc[e] = 0.f;
-#pragma nounroll
-        for (int a0 = 0; a0 < p.nasm; a0 += G) {
-          asm_x_put<N, TPW>(p, lds + wave * TPW * LP, rows, a0 + wave * TPW, lane);
-          // the next (plane, round) this wavefront loads
-          int na0 = a0 + G, nz = zout;
-          if (na0 >= p.nasm) {
-            na0 = 0;
-            ++nz;
-          }
-          if (nz < p.zdim) asm_x_fetch<N, TPW>(p, rows, na0 + wave * TPW, nz, Y, lane);
-          wave_lds_sync();
-          fft2_lds<N, true, true>(lds + g * LP, t, twt);
-          __syncthreads();
-          if (a0 == 0)
-            asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, 0>(p, lds, a0, Y, acc, lut);
-          else if (a0 == G)
-            asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, 1>(p, lds, a0, Y, acc, lut);
-          else
-            asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, -1>(p, lds, a0, Y, acc, lut);
-          __syncthreads();
-        }
-        float* orow = p.out + ((long long)zout * p.ydim + Y) * N;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const int X = threadIdx.x + e * NT;
-          if (X < N) orow[X] = acc[e];
-        }
-      }
-      return;
+      const float ky = (float)y * p.dky;
+      live = live && ky * ky <= ymax2;
+      const float2 t = src[(long long)(live ? y + hy : hy) * p.nx];
+      in[c * N1 + n1] = live ? t : make_float2(0.f, 0.f);
     }
   }
-  for (int zout = 0; zout < p.zdim; ++zout) {
-    float acc[E];
+  float2 out[N2];
+  rp_transform<LEN, HALVES, true, false>(buf + (w + (odd ? W : 0)) * C::span_of(W), j, odd, tw, in, out);
+  if (xc0 + w < p.nx && (K::ROWS == K::T || j < K::ROWS)) {
+    float2* dcol = dst + (long long)K::out0(j, odd ? 1 : 0) * p.nx + xc0 + w;
 #pragma unroll
-    for (int e = 0; e < E; ++e) acc[e] = 0.f;
-#pragma nounroll
-    for (int a0 = 0; a0 < p.nasm; a0 += G) {
-      if constexpr (asm_x_fft2<N>()) {
-        // each wavefront loads and transforms its own TPW bands, so only the
-        // accumulation below needs the whole workgroup
-        constexpr int TPW = 64 / TPT;
-        const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-        asm_x_load_rows<N, TPW>(p, lds + wave * TPW * LP, a0 + wave * TPW, zout, Y, lane);
-        wave_lds_sync();
-        fft2_lds<N, true, true>(lds + g * LP, t, twt);
-        __syncthreads();
-      } else {
-        // G bands of row Y of plane zout, zero-padded to N, into LDS
-        for (int idx = threadIdx.x; idx < G * N; idx += NT) {
-          const int sl = idx / N, X = idx - sl * N;
-          const int a = a0 + sl;
-          float2 v = make_float2(0.f, 0.f);
-          if (a < p.nasm) {
-            int x;
-            bool valid = true;
-            if (X <= p.nx - half)
-              x = X;
-            else if (X >= N - (half - 1))
-              x = X - N;
-            else {
-              x = 0;
-              valid = false;
-            }
-            if (valid) v = p.stageY[(((long long)a * p.zdim + zout) * p.ydim + Y) * p.nx + (x + (half - 1))];
-          }
-          lds[sl * LP + asm_x_pos<N>(X)] = v;
-        }
-        __syncthreads();
-        fft_lds_t<N, true, TPT>(lds + g * LP, t, twt);
-      }
-      if (a0 == 0)
-        asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, 0>(p, lds, a0, Y, acc, lut);
-      else if (a0 == G)
-        asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, 1>(p, lds, a0, Y, acc, lut);
-      else
-        asm_x_round<N, NT, G, E, LB, LUT ? LB : 0, -1>(p, lds, a0, Y, acc, lut);
-      __syncthreads();
-    }
-    float* orow = p.out + ((long long)zout * p.ydim + Y) * N;
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int X = threadIdx.x + e * NT;
-      if (X < N) orow[X] = acc[e];
-    }
+    for (int k2 = 0; k2 < N2; ++k2) dcol[(long long)(K::OSTEP * k2) * p.nx] = out[k2];
   }
 }
 
@@ -994,16 +480,25 @@ void launch_asm_z(const AsmParams& p, hipStream_t s) {
   }
 }
 
-void launch_asm_y(const AsmParams& p, hipStream_t s) {
+// The y pass at zoomed height N; run = false only requests its twiddle table.
+template <int N, int HALVES>
+static void launch_asm_y_n(const AsmParams& p, bool run, hipStream_t s) {
+  using C = AsmY<N, HALVES>;
+  const float2* tw = twiddles_rp(N, C::K::N2);
+  if (!run) return;
+  hipLaunchKernelGGL((k_asm_y<N, HALVES>), dim3(ceil_div(p.nx, C::W), p.zdim, p.nasm), dim3(C::NT), 0, s, p, tw);
+  SIMR_LAUNCH_CHECK();
+}
+
+static void asm_y_dispatch(const AsmParams& p, bool run, hipStream_t s) {
   switch (p.ydim) {
-#define SIMR_CASE(N)                                                                                \
-  case N: {                                                                                         \
-    constexpr int W = asm_y_w<N>();                                                                 \
-    hipLaunchKernelGGL(k_asm_y<N>, dim3(ceil_div(p.nx, W), p.zdim, p.nasm), dim3(W * asm_y_tpt<N>()), \
-                       0, s, p, twiddles(N));                                                       \
-    SIMR_LAUNCH_CHECK();                                                                            \
-    return;                                                                                         \
-  }
+#define SIMR_CASE(N)                            \
+  case N:                                       \
+    if (2 * p.ny == N)                          \
+      launch_asm_y_n<N, 2>(p, run, s);          \
+    else                                        \
+      launch_asm_y_n<N, 1>(p, run, s);          \
+    return;
     SIMR_ZOOM_SIZES(SIMR_CASE)
 #undef SIMR_CASE
     default:
@@ -1011,19 +506,7 @@ void launch_asm_y(const AsmParams& p, hipStream_t s) {
   }
 }
 
-void launch_asm_x(const AsmParams& p, hipStream_t s) {
-  switch (p.xdim) {
-#define SIMR_CASE(N)                                                                                       \
-  case N:                                                                                                  \
-    hipLaunchKernelGGL(k_asm_x<N>, dim3(p.ydim), dim3(asm_x_threads<N>()), 0, s, p,                    \
-                       twiddles(N));                                                                       \
-    SIMR_LAUNCH_CHECK();                                                                                   \
-    return;
-    SIMR_ZOOM_SIZES(SIMR_CASE)
-#undef SIMR_CASE
-    default:
-      throw ArgError("zoomed width " + std::to_string(p.xdim) + " is not a supported size");
-  }
-}
+void asm_y_request_tables(const AsmParams& p) { asm_y_dispatch(p, false, nullptr); }
+void launch_asm_y(const AsmParams& p, hipStream_t s) { asm_y_dispatch(p, true, s); }
 
 }  // namespace simr

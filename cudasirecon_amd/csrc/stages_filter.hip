@@ -350,15 +350,4 @@ void launch_filter_batch(const FilterParams& p, const FilterBatch& b, hipStream_
   SIMR_LAUNCH_CHECK();
 }
 
-__global__ void k_zero(float2* __restrict__ p, long long n) {
-  const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (e < n) p[e] = make_float2(0.f, 0.f);
-}
-
-void launch_zero(float2* p, long long n, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_zero, dim3(ceil_div(n, 256)), dim3(256), 0, s, p, n);
-  SIMR_LAUNCH_CHECK();
-}
-
 }  // namespace simr

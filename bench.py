@@ -41,9 +41,9 @@ KERNEL_OF_STAGE = {
     "ov_y": "simr::k_fft2_cols<{ny}, true, ...>",
     "ov_zsum": "simr::k_overlaps_zsum<false, false>",
     "ov_cols": "simr::k_ovf_cols<{ny}, true>",
-    "ov_rows": "simr::k_ovf_rows<{nx}> + simr::k_zsum_totals",
+    "ov_rows": "simr::k_ovf_rows<{nx}>",
     "modamp": "simr::k_modamp_fp64",
-    "findk0_peak": "simr::k_cc_prep + 2D FFT + simr::k_argmax_*",
+    "findk0_peak": "2D FFT + simr::k_argmax_partial + simr::k_fit_begin",
     "filter": "simr::k_filter<...> (every band of the stack)",
     "asm_z": "simr::k_asm_z_pair<{zdim}, true> + simr::k_asm_z_pair<{zdim}, false>",
     "asm_y": "simr::k_asm_y<{ydim}, ...>",

@@ -133,6 +133,42 @@ __device__ __forceinline__ float2 cmul_nc(float2 a, float2 b) {
   return make_float2(re, im);
 }
 
+// The sum of get(0 .. n-1) by one wavefront: lane l adds l, l + 64, ... in
+// order, then the lanes' sums meet pairwise (the same value in every lane).
+// Every reader of the z sums' totals adds their partials this way, and every
+// reader of the modamp partials by quad_sum, so the paths agree bit for bit.
+__device__ __forceinline__ double wave_total(double v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  return v;
+}
+template <typename Get>
+__device__ __forceinline__ double wave_sum(int n, Get get) {
+  double acc = 0.0;
+#pragma unroll 4
+  for (int i = threadIdx.x & 63; i < n; i += 64) acc += get(i);
+  return wave_total(acc);
+}
+
+// The sums of the .x and (*y) .y of get(0 .. n-1) by four neighbouring lanes:
+// lane q of the four adds q, q + 4, ... in order, then the four meet pairwise.
+template <typename Get>
+__device__ __forceinline__ double quad_sum(int n, Get get, double* y) {
+  double ax = 0.0, ay = 0.0;
+#pragma unroll 8
+  for (int i = threadIdx.x & 3; i < n; i += 4) {
+    const double2 v = get(i);
+    ax += v.x;
+    ay += v.y;
+  }
+  ax += __shfl_xor(ax, 1);
+  ay += __shfl_xor(ay, 1);
+  ax += __shfl_xor(ax, 2);
+  ay += __shfl_xor(ay, 2);
+  *y = ay;
+  return ax;
+}
+
 template <int BS>
 __device__ __forceinline__ double block_sum_d(double v, double* red) {
   const int tid = threadIdx.x;

@@ -698,7 +698,7 @@ OvParams Engine::ov_params(int dir, int o1, int o2, float k0x, float k0y) const 
 // makeoverlaps (gpuFunctionsImpl.cu:497-675) for every request, at most one
 // per direction, each in its direction's slot (or all in `only`, the dumps'
 // scratch, for a single request): one launch per pass covers every request.
-void Engine::make_overlaps(const std::vector<OvReq>& reqs, bool per_elem, FitWork* only) {
+void Engine::make_overlaps(const std::vector<OvReq>& reqs, bool per_elem, FitWork* only, bool want_cc) {
   SIMR_REQUIRE(!reqs.empty() && (int)reqs.size() <= kMaxDirs && (!only || reqs.size() == 1),
                "overlap batch: 1..8 requests");
   OvBatch b{};
@@ -723,6 +723,7 @@ void Engine::make_overlaps(const std::vector<OvReq>& reqs, bool per_elem, FitWor
     z.SX[k] = w.SX;
     z.SY[k] = w.SY;
     z.totals[k] = w.sumparts;
+    z.cc[k] = want_cc ? w.cc : nullptr;
     z.nzs[k] = 2 * b.p[k].zd + 1;
     w.zd = b.p[k].zd;
     w.cache.clear();
@@ -730,7 +731,9 @@ void Engine::make_overlaps(const std::vector<OvReq>& reqs, bool per_elem, FitWor
     dmax = std::max(dmax, r.dir);
   }
   // the FP64 fit's overlaps in two passes where the sizes allow
-  if (!only && !per_elem && !fit_fp32_ && fused_ov_ && overlaps_fused_ok(b, z)) {
+  const bool fused = !only && !per_elem && !fit_fp32_ && fused_ov_ && overlaps_fused_ok(b, z);
+  for (const OvReq& r : reqs) (only ? *only : fw_[r.dir]).zb = fused ? L.ny : zsum_blocks(L.nxy);
+  if (fused) {
     int st = stage_begin("ov_cols", stream_);
     launch_overlaps_fused_cols(b, stream_);
     stage_end(st, stream_);
@@ -762,6 +765,7 @@ ModampSlots Engine::modamp_slots() const {
     m.SX[d] = fw_[d].SX;
     m.SY[d] = fw_[d].SY;
     m.totals[d] = fw_[d].sumparts;
+    m.zb[d] = fw_[d].zb;
   }
   return m;
 }
@@ -792,7 +796,7 @@ void Engine::eval_enqueue(const Cand* c, int n, int at) {
     launch_modamp_fp32(m, cs, n, L.nx, L.ny, P.dxy, part32_, stream_);
   else
     launch_modamp_fp64(m, cs, n, L.nx, L.ny, P.dxy, part64_, stream_);
-  launch_modamp_evals(fit_fp32_, m, cs, n, part64_, part32_, nb, zsum_blocks(L.nxy), dev, true, stream_);
+  launch_modamp_evals(fit_fp32_, m, cs, n, part64_, part32_, nb, dev, true, stream_);
   stage_end(st, stream_);
 }
 
@@ -935,14 +939,11 @@ void Engine::findk0_all(const std::vector<int>& dirs) {
     dmin = std::min(dmin, d);
     dmax = std::max(dmax, d);
   }
-  make_overlaps(reqs);
+  make_overlaps(reqs, false, nullptr, true);
   // the cross-correlations of directions dmin..dmax, one after another
-  PeakBatch pb{};
-  pb.n = dmax - dmin + 1;
-  for (int k = 0; k < pb.n; ++k) pb.P[k] = fw_[dmin + k].P;
   const int st = stage_begin("findk0_peak", stream_);
   // the peak values and indices land in the zero-copy region
-  launch_findpeak(pb, fw_[dmin].cc, pv_, pi_, (float*)(dzc_ + kZcPeakV), (int*)(dzc_ + kZcPeakI), L.nx, L.ny,
+  launch_findpeak(dmax - dmin + 1, fw_[dmin].cc, pv_, pi_, (float*)(dzc_ + kZcPeakV), (int*)(dzc_ + kZcPeakI), L.nx, L.ny,
                   stream_);
   stage_end(st, stream_);
   wait_fit();
@@ -1190,41 +1191,7 @@ bool Engine::fit_on_device() {
   a.deltaangle = 0.001f;
   a.deltamag = (float)(0.1 / (double)((float)std::max(L.nx, L.ny) * P.dxy));
   for (int d = 0; d < L.ndirs; ++d) a.guess[d] = k0_[d];
-  // findk0's overlaps at the guesses and their cross-correlation peaks
-  std::vector<OvReq> reqs;
-  for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, 0, fo2, k0_[d].x, k0_[d].y});
-  make_overlaps(reqs);
-  PeakBatch pb{};
-  pb.n = L.ndirs;
-  for (int k = 0; k < pb.n; ++k) pb.P[k] = fw_[k].P;
-  int st = stage_begin("findk0_peak", stream_);
-  launch_findpeak(pb, fw_[0].cc, pv_, pi_, fitst_->peak_vals, fitst_->peak_idx, L.nx, L.ny, stream_);
-  launch_fit_start(fitst_, a, stream_);
-  stage_end(st, stream_);
-  // the fit's overlaps at every direction's start vector, then the rounds
-  reqs.clear();
-  for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, 0, fo2, 0.f, 0.f, &fitst_->d[d].kov, (float)fo2});
-  make_overlaps(reqs);
-  const ModampSlots ms = modamp_slots();
-  launch_fit_walk(fitst_, a, amps_dev_, corr_dev_, stream_);
-  CandSet cs{};
-  cs.kc = fitst_->kc;
-  cs.ks = fitst_->ks;
-  cs.nd = &fitst_->ncand;
-  const int np = fit_fp32_ ? modamp_partials_fp32(L.nx, L.ny) : modamp_partials_fp64(L.nx, L.ny);
-  const int rounds = fit_rounds_;
-  for (int r = 0; r < rounds; ++r) {
-    st = stage_begin("modamp", stream_);
-    if (fit_fp32_)
-      launch_modamp_fp32(ms, cs, kFitReq * L.ndirs, L.nx, L.ny, P.dxy, part32_, stream_);
-    else
-      launch_modamp_fp64(ms, cs, kFitReq * L.ndirs, L.nx, L.ny, P.dxy, part64_, stream_);
-    launch_modamp_evals(fit_fp32_, ms, cs, kFitReq * L.ndirs, part64_, part32_, np, zsum_blocks(L.nxy),
-                        &fitst_->ev[0][0], false, stream_);
-    launch_fit_walk(fitst_, a, amps_dev_, corr_dev_, stream_);
-    stage_end(st, stream_);
-  }
-  // the other orders' modamps at the fitted k0 (as fitk0_all)
+  // the other orders, fitted at the fitted k0 (as fitk0_all)
   std::vector<std::pair<int, int>> others;
   if (L.nz == 1) {
     for (int order = 2; order < L.norders; ++order) others.push_back({order - 1, order});
@@ -1232,16 +1199,57 @@ bool Engine::fit_on_device() {
     for (int order = 1; order < L.norders; ++order)
       if (order != fo2) others.push_back({0, order});
   }
-  const int nparts = fit_fp32_ ? modamp_partials_fp32(L.nx, L.ny) : modamp_partials_fp64(L.nx, L.ny);
   for (auto& oo : others) {
-    const float mult = (float)(oo.second - oo.first);
+    a.kc[a.nothers] = kc_dev_ + (size_t)oo.second * L.ndirs;
+    a.kmul[a.nothers++] = (float)(oo.second - oo.first);
+  }
+  // the kernel that completes the results publishes them: the last other
+  // order's, or the last walker step
+  FitPub pub{};
+  pub.ndirs = L.ndirs;
+  pub.norders = L.norders;
+  pub.out = (FitOut*)(dzc_ + kZcFit);
+  pub.flag = (unsigned*)(dzc_ + kZcFlag);
+  const unsigned seq = ++fit_seq_;
+  pub.seq = seq;
+  const FitPub nopub{};
+  // findk0's overlaps at the guesses and their cross-correlation peaks
+  std::vector<OvReq> reqs;
+  for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, 0, fo2, k0_[d].x, k0_[d].y});
+  make_overlaps(reqs, false, nullptr, true);
+  int st = stage_begin("findk0_peak", stream_);
+  launch_peak_partials(L.ndirs, fw_[0].cc, pv_, pi_, L.nx, L.ny, stream_);
+  launch_fit_begin(fitst_, a, fw_[0].cc, pv_, pi_, stream_);
+  stage_end(st, stream_);
+  // the fit's overlaps at every direction's start vector, then the rounds
+  reqs.clear();
+  for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, 0, fo2, 0.f, 0.f, &fitst_->d[d].kov, (float)fo2});
+  make_overlaps(reqs);
+  const ModampSlots ms = modamp_slots();
+  CandSet cs{};
+  cs.kc = fitst_->kc;
+  cs.nreq = fitst_->nreq;
+  const int np = fit_fp32_ ? modamp_partials_fp32(L.nx, L.ny) : modamp_partials_fp64(L.nx, L.ny);
+  const int rounds = fit_rounds_;
+  for (int r = 0; r < rounds; ++r) {
+    st = stage_begin("modamp", stream_);
+    if (fit_fp32_) {
+      launch_modamp_fp32(ms, cs, kFitReq * L.ndirs, L.nx, L.ny, P.dxy, part32_, stream_);
+      launch_modamp_evals(true, ms, cs, kFitReq * L.ndirs, part64_, part32_, np, &fitst_->ev[0][0], false, stream_);
+    } else {
+      launch_modamp_fp64(ms, cs, kFitReq * L.ndirs, L.nx, L.ny, P.dxy, part64_, stream_);
+    }
+    launch_fit_walk(fitst_, a, ms, part64_, np, amps_dev_, corr_dev_,
+                    r + 1 == rounds && others.empty() ? pub : nopub, stream_);
+    stage_end(st, stream_);
+  }
+  for (size_t i = 0; i < others.size(); ++i) {
+    const auto& oo = others[i];
     reqs.clear();
-    for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, oo.first, oo.second, 0.f, 0.f, &fitst_->d[d].kov, mult});
+    for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, oo.first, oo.second, 0.f, 0.f, &fitst_->d[d].kov, a.kmul[i]});
     make_overlaps(reqs);
-    float2* kc = kc_dev_ + (size_t)oo.second * L.ndirs;
-    launch_fit_kc(fitst_, L.ndirs, mult, kc, stream_);
     CandSet c2{};
-    c2.kc = kc;
+    c2.kc = a.kc[i];
     c2.ks = slot_ids_;
     st = stage_begin("modamp", stream_);
     const ModampSlots m = modamp_slots();
@@ -1249,13 +1257,10 @@ bool Engine::fit_on_device() {
       launch_modamp_fp32(m, c2, L.ndirs, L.nx, L.ny, P.dxy, part32_, stream_);
     else
       launch_modamp_fp64(m, c2, L.ndirs, L.nx, L.ny, P.dxy, part64_, stream_);
-    launch_modamp_finish(fit_fp32_, m, slot_ids_, L.ndirs, part64_, part32_, nparts, zsum_blocks(L.nxy), amps_dev_,
-                         corr_dev_, L.norders, oo.second, stream_);
+    launch_modamp_finish(fit_fp32_, m, slot_ids_, L.ndirs, part64_, part32_, np, amps_dev_, corr_dev_, L.norders,
+                         oo.second, fitst_, i + 1 == others.size() ? pub : nopub, stream_);
     stage_end(st, stream_);
   }
-  FitOut* out = (FitOut*)(dzc_ + kZcFit);
-  const unsigned seq = ++fit_seq_;
-  launch_fit_publish(fitst_, a, amps_dev_, corr_dev_, out, (unsigned*)(dzc_ + kZcFlag), seq, stream_);
   wait_flag(seq);
   const FitOut& o = *(const FitOut*)(hzc_ + kZcFit);
   if (o.overflow || o.ndone < L.ndirs) {
@@ -1573,8 +1578,8 @@ void Engine::build_graph() {
         launch_modamp_fp32(m, cs, L.ndirs, L.nx, L.ny, P.dxy, part32_, stream_);
       else
         launch_modamp_fp64(m, cs, L.ndirs, L.nx, L.ny, P.dxy, part64_, stream_);
-      launch_modamp_finish(fit_fp32_, m, slot_ids_, L.ndirs, part64_, part32_, nparts, zsum_blocks(L.nxy),
-                           amps_dev_, corr_dev_, L.norders, o, stream_);
+      launch_modamp_finish(fit_fp32_, m, slot_ids_, L.ndirs, part64_, part32_, nparts, amps_dev_, corr_dev_,
+                           L.norders, o, nullptr, FitPub{}, stream_);
     }
     AmpPolicy a{};
     a.ndirs = L.ndirs;

@@ -102,6 +102,7 @@ class Engine {
     float2* cc = nullptr;  // [ny][nx]
     double* sumparts = nullptr;
     int zd = 0;  // z support half-width of the overlaps in ovx
+    int zb = 0;  // partials of each z-sum total in sumparts
     std::map<std::pair<uint32_t, uint32_t>, Eval> cache;
   };
   struct OvReq {
@@ -122,7 +123,9 @@ class Engine {
   OvParams ov_params(int dir, int o1, int o2, float k0x, float k0y) const;
   // builds the requested overlap pairs (each in its direction's slot, or
   // every one in `only` when given) and their z sums
-  void make_overlaps(const std::vector<OvReq>& reqs, bool per_elem = false, FitWork* only = nullptr);
+  // (want_cc: and their cross-correlations, into FitWork::cc)
+  void make_overlaps(const std::vector<OvReq>& reqs, bool per_elem = false, FitWork* only = nullptr,
+                     bool want_cc = false);
   using Cand = std::pair<int, float2>;  // (direction, candidate vector)
   ModampSlots modamp_slots() const;
   void eval_enqueue(const Cand* c, int n, int at);

@@ -88,14 +88,11 @@ void launch_overlaps_y(int nx, int ny, int nzs_stride, float2* ovx, int nslots, 
 // P = sum_z conj(X) Y, SX = sum |X|^2, SY = sum |Y|^2 (double storage).
 // fp32: accumulated in float as the reference's reductionKernel threads, P,
 // SX, SY stored per (x, y).  Otherwise in double, P per (x, y) and the totals
-// of SX and SY as zsum_blocks(nx*ny) partials each: totals[b], totals[nb + b]
-// (per_elem: SX and SY per (x, y) as well), and their sums in block order at
-// totals[kZsumFinal], totals[kZsumFinal + 1].
+// of SX and SY as nb partials each: totals[b], totals[nb + b] (per_elem: SX
+// and SY per (x, y) as well); the readers of the totals add the partials up
+// (wave_sum).  nb = zsum_blocks(nx*ny), or ny from the two-pass form.
 constexpr int kZsumMaxBlocks = 2048;
-// totals buffer of one slot: [2][kZsumMaxBlocks] block partials, then the two
-// totals summed in block order (fp64, written by the z-sum pass)
-constexpr int kZsumFinal = 2 * kZsumMaxBlocks;
-constexpr int kZsumTotals = kZsumFinal + 2;
+constexpr int kZsumTotals = 2 * kZsumMaxBlocks;  // doubles of one slot's totals buffer
 int zsum_blocks(long long nxy);
 struct ZsumBatch {
   const float2* ovx[kMaxDirs];
@@ -103,6 +100,9 @@ struct ZsumBatch {
   double* SX[kMaxDirs];
   double* SY[kMaxDirs];
   double* totals[kMaxDirs];
+  // non-null: also conj(P) in float there (the cross-correlation's input:
+  // aTimesConjB, X conj(Y) = conj(conj(X) Y))
+  float2* cc[kMaxDirs];
   int nzs[kMaxDirs];
   int n, nzs_stride, nz;
   long long nxy;
@@ -120,17 +120,15 @@ void launch_overlaps_fused_rows(const ZsumBatch& zb, int nx, int ny, hipStream_t
 // volumes vol[2][nz][nx*ny] (debug dump only).
 void launch_overlap_volumes(const float2* ovx, int zd, int nzs_stride, int nz, long long nxy, float2* vol,
                             hipStream_t s);
-// crosscorr = conj(P) as float, then its forward 2D FFT and |.|^2 argmax, for
-// n slots: cc [n][nx*ny] (contiguous), partials [n][kArgBlocks],
-// peak_vals [n][8] (the 5 intensities centre, x-1, x+1, y-1, y+1),
-// peak_idx [n] (index of the first maximum).
+// The forward 2D FFT of n cross-correlations cc [n][nx*ny] (as the z sums
+// leave them) and the per-block maxima of |.|^2, [n][kArgBlocks] (value and
+// index of the first maximum).
 constexpr int kArgBlocks = 256;
-struct PeakBatch {
-  const double2* P[kMaxDirs];
-  int n;
-};
-void launch_findpeak(const PeakBatch& b, float2* cc, float* partial_val, int* partial_idx, float* peak_vals,
-                     int* peak_idx, int nx, int ny, hipStream_t s);
+void launch_peak_partials(int n, float2* cc, float* partial_val, int* partial_idx, int nx, int ny, hipStream_t s);
+// ... and each slot's maximum: peak_vals [n][8] (the 5 intensities centre,
+// x-1, x+1, y-1, y+1), peak_idx [n].
+void launch_findpeak(int n, float2* cc, float* partial_val, int* partial_idx, float* peak_vals, int* peak_idx, int nx,
+                     int ny, hipStream_t s);
 // Modamp reductions for a batch of candidate vectors kcand[c] on slot kslot[c].
 //   fp64: out[c] = sum P e^{i phi_c} over the image in double; partials [ncand][nparts] double2.
 //   fp32: reference reductionKernel on 64x4 blocks; partials [ncand][nblocks] of
@@ -139,8 +137,11 @@ struct ModampSlots {
   const double2* P[kMaxDirs];
   const double* SX[kMaxDirs];
   const double* SY[kMaxDirs];
-  const double* totals[kMaxDirs];  // the z-sum totals (fp64 finish)
+  const double* totals[kMaxDirs];  // the z-sum totals' partials (fp64)
+  int zb[kMaxDirs];                // ... and how many of each
 };
+constexpr int kFitLook = 7;                  // steps evaluated ahead in each direction (four lanes per candidate: at most 7)
+constexpr int kFitReq = 2 * kFitLook + 1;    // candidates a direction requests in one round
 // The candidates of one batch: device arrays (kc, ks; the graph's persistent
 // ones), or, with kc == nullptr, the values themselves in the kernel
 // arguments, so that a line-search round needs no copy.
@@ -150,10 +151,10 @@ struct CandSet {
   const int* ks;
   float2 k[kArgCand];
   int slot[kArgCand];
-  // non-null: the number of candidates, read on the device (blocks of
-  // candidates at or past it do nothing); the launch covers the most there
-  // can be
-  const int* nd;
+  // non-null: a device-driven fit's round, with the candidates of direction d
+  // at kFitReq d (ks is not read): how many there are of each, read on the
+  // device (blocks of the others do nothing)
+  const int* nreq;
 };
 int modamp_partials_fp64(int nx, int ny);
 int modamp_partials_fp32(int nx, int ny);
@@ -161,14 +162,14 @@ void launch_modamp_fp64(const ModampSlots& m, const CandSet& c, int ncand, int n
                         double2* partials, hipStream_t s);
 void launch_modamp_fp32(const ModampSlots& m, const CandSet& c, int ncand, int nx, int ny, float dxy,
                         float4* partials, hipStream_t s);
-// The sums the host makes of the modamp partials (cpuReduce,
+// The sums of the modamp partials (the reference's host sum, cpuReduce,
 // gpuFunctionsImpl_hh.cu:162-180), on the device: for candidate c, its
-// partials summed in block order and, fp64, its slot's z-sum totals;
-// out[4c..4c+3] = (xr, xi, sx, sy) (fp32: the float sums).  host_out: out is
+// partials (fp64: as wave_sum; fp32: in block order) and, fp64, its slot's
+// z-sum totals; out[4c..4c+3] = (xr, xi, sx, sy) (fp32: the float sums).  host_out: out is
 // host memory, and the writes are made visible system-wide before the kernel
 // ends.
 void launch_modamp_evals(bool fp32, const ModampSlots& m, const CandSet& c, int ncand, const double2* part64,
-                         const float4* part32, int nparts, int zblocks, double* out, bool host_out, hipStream_t s);
+                         const float4* part32, int nparts, double* out, bool host_out, hipStream_t s);
 // Writes seq to *flag (host memory) once the work queued before it is done,
 // with system-scope ordering: the host polls the flag instead of an event.
 void launch_fit_signal(unsigned* flag, unsigned seq, hipStream_t s);
@@ -180,8 +181,6 @@ void launch_fit_signal(unsigned* flag, unsigned seq, hipStream_t s);
 // (angle, mag) candidates, exactly as the host does, and writes the next
 // candidates for the modamp kernels; the host queues a fixed number of
 // (evaluate, walk) rounds and reads the results once.
-constexpr int kFitLook = 6;                  // steps evaluated ahead in each direction
-constexpr int kFitReq = 2 * kFitLook + 1;    // candidates a direction requests in one round
 constexpr int kFitMaxRounds = 8;
 constexpr int kFitCache = kFitReq * (kFitMaxRounds + 1);  // evaluated candidates kept per direction
 enum { kFitAngle = 0, kFitMag = 1, kFitFinal = 2, kFitDone = 3 };
@@ -191,39 +190,33 @@ struct FitDir {
   float k0mag, k0angle;  // the walks' start
   float angle, mag;      // fitted
   int phase, started;    // walk phase; whether its first batch was requested
-  int nreq, cand0;       // candidates requested in the last round, their first index
-  float req_a[kFitReq], req_m[kFitReq];
+  float req_a[kFitReq], req_m[kFitReq];  // the last round's requests
   int n_angle_evals, n_mag_evals, n_reductions;
+  int rounds, overflow;  // rounds with a request; more candidates than the cache holds
+  int have_totals;       // sx, sy hold the z-sum totals of the fit's overlaps
+  double sx, sy;
   int ncache;
-  float ca[kFitCache], cm[kFitCache];
-  double cev[kFitCache][4];
+  float ca[kFitCache], cm[kFitCache];                        // evaluated candidates,
+  double camp2[kFitCache], cxr[kFitCache], cxi[kFitCache];   // their |modamp|^2 and sums
 };
 struct FitState {
   FitDir d[kMaxDirs];
-  float2 kc[kArgCand];  // the round's candidate vectors and their directions
-  int ks[kArgCand];
-  int ncand;
-  int ndone, rounds, overflow;
-  float peak_vals[kMaxDirs * 8];  // findk0's cross-correlation peaks
-  int peak_idx[kMaxDirs];
-  double ev[kArgCand][4];  // the round's sums (xr, xi, sx, sy) per candidate
+  // the round's candidates: direction d's nreq[d] vectors at kc[kFitReq d]
+  float2 kc[kMaxDirs * kFitReq];
+  int nreq[kMaxDirs];
+  double ev[kMaxDirs * kFitReq][4];  // fp32: the round's sums (xr, xi, sx, sy) per candidate
 };
 struct FitArgs {
   int ndirs, norders, fo2, fp32, nx, ny;
   float dkx, dky, deltaangle, deltamag;
   float2 guess[kMaxDirs];  // the k0 findk0's overlaps were built at
+  // the other orders fitted at the fitted k0: their candidate vectors
+  // kov * kmul[i], written to kc[i][ndirs] by every walker step
+  float2* kc[kMaxOrders];
+  float kmul[kMaxOrders];
+  int nothers;
 };
-// Refines every direction's cross-correlation peak into k0 (findk0,
-// gpuFunctionsImpl.cu:316-370) and sets up the walks.
-void launch_fit_start(FitState* fs, const FitArgs& a, hipStream_t s);
-// One walker step: merges the last round's sums (fs->ev) into the caches,
-// advances every direction's walks, and writes the next round's candidates.
-// A direction that finishes gets its fitted k0 (kov) and its order-fo2
-// modamp and correlation (amps / corr [dir][norders]).
-void launch_fit_walk(FitState* fs, const FitArgs& a, float2* amps, float* corr, hipStream_t s);
-// kc[d] = kov[d] * mult for every direction
-void launch_fit_kc(const FitState* fs, int ndirs, float mult, float2* kc, hipStream_t s);
-// The results for the host, into (host-mapped) out: per direction k0 (the
+// The results for the host, in host-mapped memory: per direction k0 (the
 // search's), kov (the fitted k0) and the counters, then amps and corr
 // [dir][norders], then ndone, rounds and overflow.
 struct FitOut {
@@ -233,20 +226,36 @@ struct FitOut {
   float corr[kMaxDirs * 5];
   int ndone, rounds, overflow;
 };
-// ... then writes seq into *flag (host memory) once every result is visible
-// to the host, as launch_fit_signal does.
-void launch_fit_publish(const FitState* fs, const FitArgs& a, const float2* amps, const float* corr, FitOut* out,
-                        unsigned* flag, unsigned seq, hipStream_t s);
+// Where the fit's last kernel writes the results (out null: it does not), and
+// then seq into *flag once they are visible to the host.
+struct FitPub {
+  int ndirs, norders;
+  FitOut* out;
+  unsigned* flag;
+  unsigned seq;
+};
+// The maximum of every direction's cross-correlation from its block maxima
+// (launch_peak_partials), its refinement into k0 (findk0,
+// gpuFunctionsImpl.cu:316-370) and the walks' first requests.
+void launch_fit_begin(FitState* fs, const FitArgs& a, const float2* cc, const float* partial_val,
+                      const int* partial_idx, hipStream_t s);
+// One walker step: merges the last round's sums (fp64: of the modamp
+// partials [ncand][nparts] and the slots' totals; fp32: fs->ev) into the
+// caches, advances every direction's walks, and writes the next round's
+// candidates.  A direction that finishes gets its fitted k0 (kov) and its
+// order-fo2 modamp and correlation (amps / corr [dir][norders]).
+void launch_fit_walk(FitState* fs, const FitArgs& a, const ModampSlots& m, const double2* part64, int nparts,
+                     float2* amps, float* corr, const FitPub& pub, hipStream_t s);
 // findrealspacemodamp's result (gpuFunctionsImpl.cu:1128-1147) on the device,
-// for each of ncand candidates: the partials summed in block order as the
-// host does (cpuReduce, gpuFunctionsImpl_hh.cu:162-180), then
-// modamp = XStarY / sumX and corr = |XStarY| / sqrt(sumX sumY), written to
-// amp[kslot[c] * stride + order] and corr[same].
-// fp64: part64 [ncand][nparts] and the slot's z-sum totals [2][zblocks];
-// fp32: part32 [ncand][nparts].
+// for each of ncand candidates (one per slot): the partials summed as
+// launch_modamp_evals does, then modamp = XStarY / sumX and corr =
+// |XStarY| / sqrt(sumX sumY), written to amp[kslot[c] * stride + order] and
+// corr[same].  fp64: part64 [ncand][nparts] and the slot's z-sum totals;
+// fp32: part32 [ncand][nparts].  fit/pub: a device-driven fit whose results
+// this call completes (null: none).
 void launch_modamp_finish(bool fp32, const ModampSlots& m, const int* kslot, int ncand, const double2* part64,
-                          const float4* part32, int nparts, int zblocks, float2* amp, float* corr, int stride,
-                          int order, hipStream_t s);
+                          const float4* part32, int nparts, float2* amp, float* corr, int stride, int order,
+                          const FitState* fit, const FitPub& pub, hipStream_t s);
 // The modamp policy after every order is fitted at a known k0
 // (cudaSirecon.cpp:450-491): 2D chaining amp[o] *= amp[o-1], forcemodamp
 // (raise magnitudes below the forced ones), and with fit_all_phases == 0 the

@@ -9,7 +9,7 @@
 // vectors come from the same bit-reproducible cos/sin/atan2 (dtrig.hpp), so
 // the device walks evaluate the host walks' candidates.
 #include "dtrig.hpp"
-#include "stages.hpp"
+#include "fit_device.hpp"
 
 namespace simr {
 
@@ -53,88 +53,84 @@ __device__ double fit_amp2(const double* e, int fp32) {
 
 // One direction's walker state while a walker step runs: one wavefront per
 // direction, every lane holding the same scalar state (the logic is
-// replicated across the lanes; only the cache lookups are spread over them),
-// the evaluated keys and this round's requests in LDS.
+// replicated across the lanes; the cache lookups and the requests are spread
+// over them), the evaluated candidates in LDS, private to the wavefront.
+struct WalkerLds {
+  float ka[kFitCache], km[kFitCache];                            // evaluated (angle, mag) keys
+  double amp2[kFitCache], xr[kFitCache], xi[kFitCache];          // their |modamp|^2 and sums
+  float ra[kFitReq], rm[kFitReq];                                // this round's requests
+};
 struct Walker {
-  FitDir* f;
-  float* ka;  // evaluated (angle, mag) keys [kFitCache]
-  float* km;
-  double* amp2;  // their |modamp|^2
-  int ncache;
-  float* ra;  // this round's requests [kFitReq]
-  float* rm;
-  int nreq;
-  int lane;
+  WalkerLds* l;
+  int ncache, nreq, lane;
 };
 
-__device__ void walker_sync() {
+__device__ __forceinline__ void walker_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // index of the evaluated key (a, m), or -1: the lanes test 64 keys at a time
-__device__ int walker_find(const Walker& w, float a, float m) {
+__device__ __forceinline__ int walker_find(const Walker& w, float a, float m) {
   const unsigned ua = __float_as_uint(a), um = __float_as_uint(m);
   for (int base = 0; base < w.ncache; base += 64) {
     const int i = base + w.lane;
     const int ic = i < w.ncache ? i : 0;  // an index inside the array for every lane
-    const bool hit = i < w.ncache && __float_as_uint(w.ka[ic]) == ua && __float_as_uint(w.km[ic]) == um;
+    const bool hit = i < w.ncache && __float_as_uint(w.l->ka[ic]) == ua && __float_as_uint(w.l->km[ic]) == um;
     const unsigned long long b = __ballot(hit);
     if (b != 0ull) return base + __ffsll((long long)b) - 1;
   }
   return -1;
 }
 
-// Adds (a, m) to the round's requests unless it is evaluated or already
-// requested.
-__device__ void walker_request(Walker& w, float a, float m) {
-  if (walker_find(w, a, m) >= 0) return;
+// Requests lane i's (a, m) for every i < n, in lane order, except those that
+// are evaluated or already requested (the first request of a step: nreq is
+// 0 and n at most kFitReq).
+__device__ __forceinline__ void walker_request(Walker& w, int n, float a, float m) {
   const unsigned ua = __float_as_uint(a), um = __float_as_uint(m);
-  // the requests so far (at most kFitReq < 64), one per lane
-  const int li = w.lane < kFitReq ? w.lane : 0;  // an index inside the array for every lane
-  const bool dup = w.lane < w.nreq && __float_as_uint(w.ra[li]) == ua && __float_as_uint(w.rm[li]) == um;
-  if (__ballot(dup) != 0ull) return;
-  if (w.nreq < kFitReq) {
-    if (w.lane == 0) {
-      w.ra[w.nreq] = a;
-      w.rm[w.nreq] = m;
-    }
-    walker_sync();
-    ++w.nreq;
+  bool keep = w.lane < n;
+  for (int e = 0; e < w.ncache; ++e)
+    keep = keep && !(__float_as_uint(w.l->ka[e]) == ua && __float_as_uint(w.l->km[e]) == um);
+  for (int e = 0; e < n - 1; ++e) {
+    const unsigned va = __shfl(ua, e), vm = __shfl(um, e);
+    keep = keep && !(e < w.lane && va == ua && vm == um);
   }
+  const unsigned long long mask = __ballot(keep);
+  const int at = __popcll(mask & ((1ull << w.lane) - 1ull));
+  if (keep && at < kFitReq) {
+    w.l->ra[at] = a;
+    w.l->rm[at] = m;
+  }
+  w.nreq = min(__popcll(mask), kFitReq);
+  walker_sync();
 }
 
-// kFitLook steps of a walk from `a` (angle walks vary the angle at a fixed
-// magnitude, magnitude walks the magnitude), by the float accumulation of
-// the step.
-__device__ void walker_request_walk(Walker& w, float a, float other, bool is_angle, float delta, int sign) {
+// a after n steps of +-delta, by the float accumulation of the walk
+__device__ __forceinline__ float walk_steps(float a, int n, float delta, int sign) {
 #pragma clang fp contract(off)
-  for (int m = 0; m < kFitLook; ++m) {
-    if (is_angle)
-      walker_request(w, a, other);
-    else
-      walker_request(w, other, a);
-    a = sign > 0 ? a + delta : a - delta;
-  }
+  for (int k = 0; k < kFitLook; ++k)
+    if (k < n) a = sign > 0 ? a + delta : a - delta;
+  return a;
 }
 
 // One walk of fitk0andmodamps (gpuFunctionsImpl.cu:912-983) replayed over the
 // cache: from `start` step by `delta` while the modamp magnitude grows, then
 // the parabola through the last three points.  true: *out and *nevals set;
 // false: the next kFitLook steps from the first missing value are requested.
-__device__ bool walker_replay(Walker& w, bool is_angle, float start, float other, float delta, int fp32, float* out,
-                              int* nevals) {
+__device__ __forceinline__ bool walker_replay(Walker& w, bool is_angle, float start, float other, float delta, int fp32,
+                                              float* out, int* nevals) {
 #pragma clang fp contract(off)
   int n = 0;
   int sign = +1;
   auto val = [&](float a, double* amp) {
     const int i = is_angle ? walker_find(w, a, other) : walker_find(w, other, a);
     if (i < 0) {
-      walker_request_walk(w, a, other, is_angle, delta, sign);
+      const float q = walk_steps(a, w.lane, delta, sign);
+      walker_request(w, kFitLook, is_angle ? q : other, is_angle ? other : q);
       return false;
     }
-    *amp = w.amp2[i];
+    *amp = w.l->amp2[i];
     ++n;
     return true;
   };
@@ -198,19 +194,18 @@ __device__ void fit_modamp(const double* e, int fp32, float2* m, float* cc) {
   }
 }
 
-__global__ void k_fit_start(FitState* fs, FitArgs a) {
+// What a direction carries from one walker step to the next.
+struct DirRun {
+  int ncache, nprev, phase, started, nang, nmag, nred, rounds, over, have_totals;
+  float angle, mag, k0angle, k0mag;
+  float2 kov;
+  double sx, sy;
+};
+
+// Direction d's start from its cross-correlation's five intensities v around
+// the maximum at idx.
+__device__ __forceinline__ DirRun fit_start(const FitArgs& a, int d, const float* v, int idx, float2* k0) {
 #pragma clang fp contract(off)
-  const int d = threadIdx.x;
-  if (d == 0) {
-    fs->ncand = 0;
-    fs->ndone = 0;
-    fs->rounds = 0;
-    fs->overflow = 0;
-  }
-  if (d >= a.ndirs) return;
-  FitDir& f = fs->d[d];
-  const float* v = fs->peak_vals + d * 8;
-  const int idx = fs->peak_idx[d];
   const int xc = idx % a.nx, yc = idx / a.nx;
   float2 pk;
   pk.x = fit_parabola(v[1], v[0], v[2]) + (float)xc;
@@ -222,222 +217,251 @@ __global__ void k_fit_start(FitState* fs, FitArgs a) {
   if (old.y / a.dky > pk.y + (float)(a.ny / 2)) pk.y += (float)a.ny;
   pk.x *= a.dkx / (float)a.fo2;
   pk.y *= a.dky / (float)a.fo2;
-  f.k0 = pk;
-  f.k0mag = sqrtf(pk.x * pk.x + pk.y * pk.y);
-  f.k0angle = dtrig::fatan2(pk.y, pk.x);
-  f.kov = make_float2(f.k0mag * dtrig::fcos(f.k0angle), f.k0mag * dtrig::fsin(f.k0angle));
-  f.angle = f.mag = 0.f;
-  f.phase = kFitAngle;
-  f.started = 0;
-  f.nreq = 0;
-  f.cand0 = 0;
-  f.n_angle_evals = f.n_mag_evals = f.n_reductions = 0;
-  f.ncache = 0;
+  *k0 = pk;
+  DirRun r{};
+  r.k0mag = sqrtf(pk.x * pk.x + pk.y * pk.y);
+  r.k0angle = dtrig::fatan2(pk.y, pk.x);
+  r.kov = make_float2(r.k0mag * dtrig::fcos(r.k0angle), r.k0mag * dtrig::fsin(r.k0angle));
+  r.phase = kFitAngle;
+  return r;
 }
 
-// One wavefront per direction (blockDim = 64 * ndirs).
-__global__ __launch_bounds__(64 * kMaxDirs) void k_fit_walk(FitState* fs, FitArgs a, float2* amps, float* corr) {
+// Advances direction d's walks over the cache in w.l (w.ncache entries),
+// requests what they need next, and writes the direction's state back (one
+// wavefront).
+__device__ __forceinline__ void walk_dir(FitState* fs, const FitArgs& a, int d, DirRun r, Walker& w, float2* amps,
+                                         float* corr) {
 #pragma clang fp contract(off)
-  __shared__ float ska[kMaxDirs][kFitCache], skm[kMaxDirs][kFitCache];
-  __shared__ double samp[kMaxDirs][kFitCache];
-  __shared__ float sra[kMaxDirs][kFitReq], srm[kMaxDirs][kFitReq];
-  __shared__ int snreq[kMaxDirs], sdone[kMaxDirs], sover[kMaxDirs];
-  const int d = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const bool active = d < a.ndirs;  // uniform over each wavefront
-  FitDir& f = fs->d[active ? d : 0];
-  int ncache = 0;
-  if (active) {
-    // the keys evaluated so far, then the last round's sums of this
-    // direction's requests
-    ncache = f.ncache;
-    const int nprev = f.nreq, cand0 = f.cand0;
-    const int nadd = nprev < kFitCache - ncache ? nprev : kFitCache - ncache;
-    for (int i = lane; i < ncache; i += 64) {
-      ska[d][i] = f.ca[i];
-      skm[d][i] = f.cm[i];
-      samp[d][i] = fit_amp2(f.cev[i], a.fp32);
-    }
-    for (int i = lane; i < nadd; i += 64) {
-      const int k = ncache + i;
-      const float ra = f.req_a[i], rm = f.req_m[i];
-      ska[d][k] = ra;
-      skm[d][k] = rm;
-      f.ca[k] = ra;
-      f.cm[k] = rm;
-      double e[4];
-      for (int q = 0; q < 4; ++q) e[q] = fs->ev[cand0 + i][q];
-      for (int q = 0; q < 4; ++q) f.cev[k][q] = e[q];
-      samp[d][k] = fit_amp2(e, a.fp32);
-    }
-    if (lane == 0) sover[d] = nadd < nprev ? 1 : 0;
-    ncache += nadd;
-  }
-  __syncthreads();  // the merged sums are read back below by other lanes
-  if (active) {
-    Walker w{&f, ska[d], skm[d], samp[d], ncache, sra[d], srm[d], 0, lane};
-    int phase = f.phase, started = f.started;
-    float angle = f.angle, mag = f.mag;
-    const float k0angle = f.k0angle, k0mag = f.k0mag;
-    int nang = f.n_angle_evals, nmag = f.n_mag_evals, nred = f.n_reductions;
-    float2 kov = f.kov;
-    for (int guard = 0; guard < 4; ++guard) {
-      if (phase == kFitAngle || phase == kFitMag) {
-        const bool ang = phase == kFitAngle;
-        const float s0 = ang ? k0angle : k0mag;
-        const float other = ang ? k0mag : angle;
-        const float delta = ang ? a.deltaangle : a.deltamag;
-        if (!started) {
-          // the start and the first kFitLook steps both ways in one batch
-          started = 1;
-          if (ang)
-            walker_request(w, s0, other);
-          else
-            walker_request(w, other, s0);
-          walker_request_walk(w, s0 + delta, other, ang, delta, +1);
-          walker_request_walk(w, s0 - delta, other, ang, delta, -1);
-          if (w.nreq > 0) break;
-        }
-        float r;
-        int ne = 0;
-        if (!walker_replay(w, ang, s0, other, delta, a.fp32, &r, &ne)) break;
-        if (ang) {
-          angle = r;
-          nang += ne;
-        } else {
-          mag = r;
-          nmag += ne;
-        }
-        nred += ne;
-        phase += 1;
-        started = 0;
-      } else if (phase == kFitFinal) {
-        const int i = walker_find(w, angle, mag);
-        if (i < 0) {
-          walker_request(w, angle, mag);
-          break;
-        }
-        // getmodamp at the fitted angle and magnitude: the fitted k0 and its modamp
-        kov = make_float2(mag * dtrig::fcos(angle), mag * dtrig::fsin(angle));
-        float2 m;
-        float cc;
-        fit_modamp(f.cev[i], a.fp32, &m, &cc);
-        if (lane == 0) {
-          amps[d * a.norders + a.fo2] = m;
-          corr[d * a.norders + a.fo2] = cc;
-        }
-        nred += 1;
-        phase = kFitDone;
+  for (int guard = 0; guard < 4; ++guard) {
+    if (r.phase == kFitAngle || r.phase == kFitMag) {
+      const bool ang = r.phase == kFitAngle;
+      const float s0 = ang ? r.k0angle : r.k0mag;
+      const float other = ang ? r.k0mag : r.angle;
+      const float delta = ang ? a.deltaangle : a.deltamag;
+      if (!r.started) {
+        // the start (lane 0) and the first kFitLook steps up (lanes 1 ..) and
+        // down in one batch
+        r.started = 1;
+        const int i = w.lane;
+        const float q = i == 0            ? s0
+                        : i <= kFitLook ? walk_steps(s0 + delta, i - 1, delta, +1)
+                                          : walk_steps(s0 - delta, i - 1 - kFitLook, delta, -1);
+        walker_request(w, kFitReq, ang ? q : other, ang ? other : q);
+        if (w.nreq > 0) break;
+      }
+      float v;
+      int ne = 0;
+      if (!walker_replay(w, ang, s0, other, delta, a.fp32, &v, &ne)) break;
+      if (ang) {
+        r.angle = v;
+        r.nang += ne;
       } else {
+        r.mag = v;
+        r.nmag += ne;
+      }
+      r.nred += ne;
+      r.phase += 1;
+      r.started = 0;
+    } else if (r.phase == kFitFinal) {
+      const int i = walker_find(w, r.angle, r.mag);
+      if (i < 0) {
+        walker_request(w, 1, r.angle, r.mag);
         break;
       }
-    }
-    if (lane == 0) {
-      f.ncache = ncache;
-      f.phase = phase;
-      f.started = started;
-      f.angle = angle;
-      f.mag = mag;
-      f.kov = kov;
-      f.n_angle_evals = nang;
-      f.n_mag_evals = nmag;
-      f.n_reductions = nred;
-      f.nreq = w.nreq;
-      snreq[d] = w.nreq;
-      sdone[d] = phase == kFitDone ? 1 : 0;
-    }
-    for (int i = lane; i < w.nreq; i += 64) {
-      f.req_a[i] = sra[d][i];
-      f.req_m[i] = srm[d][i];
+      // getmodamp at the fitted angle and magnitude: the fitted k0 and its modamp
+      r.kov = make_float2(r.mag * dtrig::fcos(r.angle), r.mag * dtrig::fsin(r.angle));
+      const double e[4] = {w.l->xr[i], w.l->xi[i], r.sx, r.sy};
+      float2 m;
+      float cc;
+      fit_modamp(e, a.fp32, &m, &cc);
+      if (w.lane == 0) {
+        amps[d * a.norders + a.fo2] = m;
+        corr[d * a.norders + a.fo2] = cc;
+      }
+      r.nred += 1;
+      r.phase = kFitDone;
+    } else {
+      break;
     }
   }
-  __syncthreads();
-  if (active) {
-    int c0 = 0, total = 0, done = 0, over = 0;
-    for (int j = 0; j < a.ndirs; ++j) {
-      if (j < d) c0 += snreq[j];
-      total += snreq[j];
-      done += sdone[j];
-      over |= sover[j];
-    }
-    if (lane == 0) f.cand0 = c0;
-    for (int i = lane; i < snreq[d]; i += 64) {
-      // getmodamp's vector at (angle, mag), times order2 - order1 (1093-1094)
-      const float ra = sra[d][i], rm = srm[d][i];
-      const float kx = rm * dtrig::fcos(ra), ky = rm * dtrig::fsin(ra);
-      fs->kc[c0 + i] = make_float2(kx * (float)a.fo2, ky * (float)a.fo2);
-      fs->ks[c0 + i] = d;
-    }
-    if (threadIdx.x == 0) {
-      fs->ncand = total;
-      fs->ndone = done;
-      if (over) fs->overflow = 1;
-      if (total > 0) fs->rounds += 1;
-    }
+  FitDir& f = fs->d[d];
+  if (w.lane < w.nreq) {
+    // getmodamp's vector at (angle, mag), times order2 - order1 (1093-1094)
+    const float ra = w.l->ra[w.lane], rm = w.l->rm[w.lane];
+    const float kx = rm * dtrig::fcos(ra), ky = rm * dtrig::fsin(ra);
+    fs->kc[d * kFitReq + w.lane] = make_float2(kx * (float)a.fo2, ky * (float)a.fo2);
+    f.req_a[w.lane] = ra;
+    f.req_m[w.lane] = rm;
+  }
+  if (w.lane == 0) {
+    for (int o = 0; o < a.nothers; ++o) a.kc[o][d] = make_float2(r.kov.x * a.kmul[o], r.kov.y * a.kmul[o]);
+    fs->nreq[d] = w.nreq;
+    f.ncache = w.ncache;
+    f.phase = r.phase;
+    f.started = r.started;
+    f.angle = r.angle;
+    f.mag = r.mag;
+    f.kov = r.kov;
+    f.n_angle_evals = r.nang;
+    f.n_mag_evals = r.nmag;
+    f.n_reductions = r.nred;
+    f.rounds = r.rounds + (w.nreq > 0 ? 1 : 0);
+    f.overflow = r.over;
+    f.have_totals = r.have_totals;
+    f.sx = r.sx;
+    f.sy = r.sy;
   }
 }
 
-__global__ void k_fit_kc(const FitState* fs, int ndirs, float mult, float2* kc) {
+// The cross-correlations' maxima from their block maxima, the starts, and the
+// walks' first requests (one wavefront per direction).
+__global__ __launch_bounds__(64 * kMaxDirs) void k_fit_begin(FitState* fs, FitArgs a, const float2* __restrict__ cc,
+                                                             const float* __restrict__ pv,
+                                                             const int* __restrict__ pi) {
+  __shared__ WalkerLds lds[kMaxDirs];
+  const int d = threadIdx.x / 64, lane = threadIdx.x % 64;
+  if (d >= a.ndirs) return;
+  cc += (long long)d * a.nx * a.ny;
+  pv += d * kArgBlocks;
+  pi += d * kArgBlocks;
+  float v = -1e30f;
+  int idx = 0x7fffffff;
+#pragma unroll
+  for (int b = 0; b < kArgBlocks; b += 64) better(v, idx, pv[b + lane], pi[b + lane]);
+  for (int off = 32; off > 0; off >>= 1) {
+    const float v2 = __shfl_xor(v, off);
+    const int i2 = __shfl_xor(idx, off);
+    better(v, idx, v2, i2);
+  }
+  // No element won (every intensity NaN): findpeak keeps its initial centre
+  // (gpuFunctionsImpl.cu:443-455).
+  if (idx < 0 || idx >= a.nx * a.ny) idx = 0;
+  const int xc = idx % a.nx, yc = idx / a.nx;
+  // lanes 0..4: centre, x-1, x+1, y-1, y+1, wrapped
+  int x = xc, y = yc;
+  if (lane == 1) x = xc == 0 ? a.nx - 1 : xc - 1;
+  if (lane == 2) x = xc == a.nx - 1 ? 0 : xc + 1;
+  if (lane == 3) y = yc == 0 ? a.ny - 1 : yc - 1;
+  if (lane == 4) y = yc == a.ny - 1 ? 0 : yc + 1;
+  const float in = intensity(cc[(long long)y * a.nx + x]);
+  float t[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) t[k] = __shfl(in, k);
+  float2 k0;
+  const DirRun r = fit_start(a, d, t, idx, &k0);
+  if (lane == 0) {
+    FitDir& f = fs->d[d];
+    f.k0 = k0;
+    f.k0mag = r.k0mag;
+    f.k0angle = r.k0angle;
+  }
+  Walker w{&lds[d], 0, 0, lane};
+  walk_dir(fs, a, d, r, w, nullptr, nullptr);
+}
+
+// One walker step (one wavefront per direction, blockDim = 64 * ndirs).  The
+// round's partials are loaded beside the direction's state (a direction's
+// candidates always sit at kFitReq d), four lanes to a candidate.
+__global__ __launch_bounds__(64 * kMaxDirs) void k_fit_walk(FitState* fs, FitArgs a, ModampSlots m,
+                                                            const double2* __restrict__ part64, int nparts,
+                                                            float2* amps, float* corr, FitPub pub) {
 #pragma clang fp contract(off)
-  const int d = threadIdx.x;
-  if (d >= ndirs) return;
-  const float2 k = fs->d[d].kov;
-  kc[d] = make_float2(k.x * mult, k.y * mult);
-}
-
-__global__ void k_fit_publish(const FitState* fs, FitArgs a, const float2* amps, const float* corr, FitOut* out,
-                              unsigned* flag, unsigned seq) {
-  const int t = threadIdx.x;
-  if (t < a.ndirs) {
-    const FitDir& f = fs->d[t];
-    out->k0[t] = f.k0;
-    out->kov[t] = f.kov;
-    out->n_angle_evals[t] = f.n_angle_evals;
-    out->n_mag_evals[t] = f.n_mag_evals;
-    out->n_reductions[t] = f.n_reductions;
+  __shared__ WalkerLds lds[kMaxDirs];
+  const int d = threadIdx.x / 64, lane = threadIdx.x % 64;
+  if (d < a.ndirs) {  // uniform over each wavefront
+    FitDir& f = fs->d[d];
+    WalkerLds& l = lds[d];
+    const int ci = lane / 4 < kFitReq ? lane / 4 : kFitReq - 1;  // the lane's candidate
+    double xr = 0.0, xi = 0.0;
+    if (!a.fp32) {
+      const double2* p = part64 + (long long)(d * kFitReq + ci) * nparts;
+      xr = quad_sum(nparts, [&](int i) { return p[i]; }, &xi);
+    }
+    DirRun r;
+    r.ncache = f.ncache;
+    r.nprev = fs->nreq[d];
+    r.phase = f.phase;
+    r.started = f.started;
+    r.nang = f.n_angle_evals;
+    r.nmag = f.n_mag_evals;
+    r.nred = f.n_reductions;
+    r.rounds = f.rounds;
+    r.over = f.overflow;
+    r.have_totals = f.have_totals;
+    r.angle = f.angle;
+    r.mag = f.mag;
+    r.k0angle = f.k0angle;
+    r.k0mag = f.k0mag;
+    r.kov = f.kov;
+    r.sx = f.sx;
+    r.sy = f.sy;
+    const int nadd = min(r.nprev, kFitCache - r.ncache);
+    if (nadd < r.nprev) r.over = 1;
+    // the candidates evaluated so far
+    for (int i = lane; i < r.ncache; i += 64) {
+      l.ka[i] = f.ca[i];
+      l.km[i] = f.cm[i];
+      l.amp2[i] = f.camp2[i];
+      l.xr[i] = f.cxr[i];
+      l.xi[i] = f.cxi[i];
+    }
+    if (nadd > 0) {
+      if (a.fp32) {
+        const double* e = fs->ev[d * kFitReq + ci];
+        xr = e[0];
+        xi = e[1];
+        r.sx = fs->ev[d * kFitReq][2];  // the same for every candidate of a direction
+        r.sy = fs->ev[d * kFitReq][3];
+      } else if (!r.have_totals) {
+        const int zb = m.zb[d];
+        const double* t = m.totals[d];
+        r.sx = wave_sum(zb, [&](int i) { return t[i]; });
+        r.sy = wave_sum(zb, [&](int i) { return t[zb + i]; });
+        r.have_totals = 1;
+      }
+      // the round's candidates join them
+      if (lane % 4 == 0 && lane / 4 < nadd) {
+        const int k = r.ncache + ci;
+        const double e[4] = {xr, xi, r.sx, r.sy};
+        const double amp2 = fit_amp2(e, a.fp32);
+        const float ra = f.req_a[ci], rm = f.req_m[ci];
+        l.ka[k] = f.ca[k] = ra;
+        l.km[k] = f.cm[k] = rm;
+        l.amp2[k] = f.camp2[k] = amp2;
+        l.xr[k] = f.cxr[k] = xr;
+        l.xi[k] = f.cxi[k] = xi;
+      }
+    }
+    walker_sync();
+    Walker w{&l, r.ncache + nadd, 0, lane};
+    walk_dir(fs, a, d, r, w, amps, corr);
   }
-  for (int i = t; i < a.ndirs * a.norders; i += blockDim.x) {
-    out->amps[i] = amps[i];
-    out->corr[i] = corr[i];
+  if (pub.out != nullptr) {
+    __syncthreads();
+    fit_publish(fs, pub, amps, corr);
   }
-  if (t == 0) {
-    out->ndone = fs->ndone;
-    out->rounds = fs->rounds;
-    out->overflow = fs->overflow;
-  }
-  __threadfence_system();  // out is host memory
-  __syncthreads();
-  if (t == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 void check_fit_args(const FitArgs& a) {
-  if (a.ndirs < 1 || a.ndirs > kMaxDirs || a.norders < 1 || a.norders > 5 || a.fo2 < 1 || a.fo2 >= a.norders ||
+  if (a.ndirs < 1 || a.ndirs > kMaxDirs || a.norders < 1 || a.norders > 5 || a.fo2 < 1 || a.fo2 >= a.norders || a.nothers < 0 ||
+      a.nothers > kMaxOrders ||
       kFitReq * a.ndirs > kArgCand)
     throw ArgError("device fit: 1..8 directions, 2..5 orders");
 }
 
 }  // namespace
 
-void launch_fit_start(FitState* fs, const FitArgs& a, hipStream_t s) {
+void launch_fit_begin(FitState* fs, const FitArgs& a, const float2* cc, const float* partial_val,
+                      const int* partial_idx, hipStream_t s) {
   check_fit_args(a);
-  hipLaunchKernelGGL(k_fit_start, dim3(1), dim3(64), 0, s, fs, a);
+  hipLaunchKernelGGL(k_fit_begin, dim3(1), dim3(64 * a.ndirs), 0, s, fs, a, cc, partial_val, partial_idx);
   SIMR_LAUNCH_CHECK();
 }
 
-void launch_fit_walk(FitState* fs, const FitArgs& a, float2* amps, float* corr, hipStream_t s) {
+void launch_fit_walk(FitState* fs, const FitArgs& a, const ModampSlots& m, const double2* part64, int nparts,
+                     float2* amps, float* corr, const FitPub& pub, hipStream_t s) {
   check_fit_args(a);
-  hipLaunchKernelGGL(k_fit_walk, dim3(1), dim3(64 * a.ndirs), 0, s, fs, a, amps, corr);
-  SIMR_LAUNCH_CHECK();
-}
-
-void launch_fit_kc(const FitState* fs, int ndirs, float mult, float2* kc, hipStream_t s) {
-  hipLaunchKernelGGL(k_fit_kc, dim3(1), dim3(64), 0, s, fs, ndirs, mult, kc);
-  SIMR_LAUNCH_CHECK();
-}
-
-void launch_fit_publish(const FitState* fs, const FitArgs& a, const float2* amps, const float* corr, FitOut* out,
-                        unsigned* flag, unsigned seq, hipStream_t s) {
-  check_fit_args(a);
-  hipLaunchKernelGGL(k_fit_publish, dim3(1), dim3(64), 0, s, fs, a, amps, corr, out, flag, seq);
+  hipLaunchKernelGGL(k_fit_walk, dim3(1), dim3(64 * a.ndirs), 0, s, fs, a, m, part64, nparts, amps, corr, pub);
   SIMR_LAUNCH_CHECK();
 }
 

@@ -24,6 +24,7 @@
 #include "fft.hpp"
 #include "fft2.hpp"
 #include "fft_api.hpp"
+#include "fit_device.hpp"
 #include "sizes.hpp"
 #include "stages.hpp"
 
@@ -338,8 +339,6 @@ void launch_overlaps_x(const OvBatch& b, hipStream_t s) {
   }
 }
 
-__global__ __launch_bounds__(256) void k_zsum_totals(ZsumBatch b, int zblocks);
-
 // ---------------------------------------------------------------------------
 // The overlaps' inverse transforms with the z sums fused, for the FP64 fit:
 // the formation runs with the y transform, by columns (k_ovf_cols), and the
@@ -547,7 +546,9 @@ __global__ __launch_bounds__(2 * kOvfG * fft_tpt(NX)) void k_ovf_rows(ZsumBatch 
   for (int e = 0; e < EPT; ++e) {
     const int x = tid + e * NT;
     if (x < NX) {
-      Pout[x] = make_double2(sxr[e] * n, sxi[e] * n);
+      const double2 pv = make_double2(sxr[e] * n, sxi[e] * n);
+      Pout[x] = pv;
+      if (b.cc[slot]) b.cc[slot][(long long)y * NX + x] = make_float2((float)pv.x, -(float)pv.y);
       tsx += sx[e] * n;
       tsy += sy[e] * n;
     }
@@ -584,8 +585,6 @@ static bool ovf_rows_launch(const ZsumBatch& zb, int ny, bool run, hipStream_t s
   if constexpr (ovf_rows_ok<NX>()) {
     if (!run) return true;
     hipLaunchKernelGGL(k_ovf_rows<NX>, dim3(ny, zb.n), dim3(2 * kOvfG * fft_tpt(NX)), 0, s, zb, twiddles(NX));
-    SIMR_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_zsum_totals, dim3(zb.n), dim3(256), 0, s, zb, ny);
     SIMR_LAUNCH_CHECK();
     return true;
   } else {
@@ -709,7 +708,9 @@ __global__ __launch_bounds__(256) void k_overlaps_zsum(ZsumBatch b) {
         }
       }
     }
-    P[e] = make_double2((double)(sxr * n), (double)(sxi * n));
+    const double2 pv = make_double2((double)(sxr * n), (double)(sxi * n));
+    P[e] = pv;
+    if (b.cc[slot]) b.cc[slot][e] = make_float2((float)pv.x, -(float)pv.y);
     if constexpr (FP32 || ELEM) {
       SX[e] = (double)(sx * n);
       SY[e] = (double)(sy * n);
@@ -730,14 +731,6 @@ __global__ __launch_bounds__(256) void k_overlaps_zsum(ZsumBatch b) {
   }
 }
 
-// The two z-sum totals of each slot (blockIdx.x), summed in block order.
-__global__ __launch_bounds__(256) void k_zsum_totals(ZsumBatch b, int zblocks) {
-  __shared__ double stage[2 * kSeqChunk];
-  double* t = b.totals[blockIdx.x];
-  const double v = seq_sum_lanes<double, 2>(zblocks, stage, [&](int i, int k) { return t[k * zblocks + i]; });
-  if (threadIdx.x < 2) t[kZsumFinal + threadIdx.x] = v;
-}
-
 void launch_overlaps_z_reduce(const ZsumBatch& b, bool fp32, bool per_elem, hipStream_t s) {
   if (b.n < 1 || b.n > kMaxDirs) throw ArgError("z-sum batch: 1..8 slots");
   for (int k = 0; k < b.n; ++k)
@@ -751,35 +744,9 @@ void launch_overlaps_z_reduce(const ZsumBatch& b, bool fp32, bool per_elem, hipS
   else
     hipLaunchKernelGGL((k_overlaps_zsum<false, false>), grid, dim3(256), 0, s, b);
   SIMR_LAUNCH_CHECK();
-  if (!fp32) {
-    hipLaunchKernelGGL(k_zsum_totals, dim3(b.n), dim3(256), 0, s, b, (int)grid.x);
-    SIMR_LAUNCH_CHECK();
-  }
 }
 
 // ----------------------------------------------------------------- findk0 peak
-__global__ void k_cc_prep(PeakBatch b, float2* __restrict__ cc, long long n) {
-  const double2* __restrict__ P = b.P[blockIdx.y];
-  cc += (long long)blockIdx.y * n;
-  long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) {
-    const double2 v = P[e];
-    cc[e] = make_float2((float)v.x, -(float)v.y);  // aTimesConjB: X conj(Y) = conj(conj(X) Y)
-  }
-}
-
-__device__ __forceinline__ void better(float& v, int& i, float v2, int i2) {
-  if (v2 > v || (v2 == v && i2 < i)) {
-    v = v2;
-    i = i2;
-  }
-}
-
-__device__ __forceinline__ float intensity(float2 a) {
-#pragma clang fp contract(off)
-  return a.x * a.x + a.y * a.y;
-}
-
 __global__ __launch_bounds__(256) void k_argmax_partial(const float2* __restrict__ cc, long long n,
                                                         float* __restrict__ pv, int* __restrict__ pi) {
   cc += (long long)blockIdx.y * n;
@@ -855,149 +822,227 @@ __global__ __launch_bounds__(256) void k_argmax_final(const float2* __restrict__
   __threadfence_system();  // the outputs may be host memory
 }
 
-void launch_findpeak(const PeakBatch& b, float2* cc, float* partial_val, int* partial_idx, float* peak_vals,
-                     int* peak_idx, int nx, int ny, hipStream_t s) {
-  if (b.n < 1 || b.n > kMaxDirs) throw ArgError("peak batch: 1..8 slots");
-  const long long n = (long long)nx * ny;
-  hipLaunchKernelGGL(k_cc_prep, dim3(ceil_div(n, 256), b.n), dim3(256), 0, s, b, cc, n);
+void launch_peak_partials(int n, float2* cc, float* partial_val, int* partial_idx, int nx, int ny, hipStream_t s) {
+  if (n < 1 || n > kMaxDirs) throw ArgError("peak batch: 1..8 slots");
+  const long long nxy = (long long)nx * ny;
+  fft_rows(nx, cc, nx, (long long)ny * n, false, s);
+  fft_cols(ny, cc, nx, nx, n, nxy, false, s);
+  hipLaunchKernelGGL(k_argmax_partial, dim3(kArgBlocks, n), dim3(256), 0, s, cc, nxy, partial_val, partial_idx);
   SIMR_LAUNCH_CHECK();
-  fft_rows(nx, cc, nx, (long long)ny * b.n, false, s);
-  fft_cols(ny, cc, nx, nx, b.n, n, false, s);
-  hipLaunchKernelGGL(k_argmax_partial, dim3(kArgBlocks, b.n), dim3(256), 0, s, cc, n, partial_val, partial_idx);
-  SIMR_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_argmax_final, dim3(b.n), dim3(256), 0, s, cc, partial_val, partial_idx, kArgBlocks, nx, ny,
+}
+
+void launch_findpeak(int n, float2* cc, float* partial_val, int* partial_idx, float* peak_vals, int* peak_idx, int nx,
+                     int ny, hipStream_t s) {
+  launch_peak_partials(n, cc, partial_val, partial_idx, nx, ny, s);
+  hipLaunchKernelGGL(k_argmax_final, dim3(n), dim3(256), 0, s, cc, partial_val, partial_idx, kArgBlocks, nx, ny,
                      peak_vals, peak_idx);
   SIMR_LAUNCH_CHECK();
 }
 
 // ------------------------------------------------------------ modamp, FP64
 // e^{i phi} = e^{i a(x)} e^{i b(y)} with a = 2 pi dxy (x - nx/2) kx and
-// b = 2 pi dxy (y - ny/2) ky: one table of nx phasors per candidate.
-constexpr int kModRows = 4;
-
+// b = 2 pi dxy (y - ny/2) ky, so
+//   sum P e^{i phi} = sum_x e^{i a(x)} sum_y e^{i b(y)} P(x, y).
+// Workgroup (row block, group of up to G candidates of one slot): a thread
+// takes columns x, adds the block's rows up with each candidate's row phasors
+// (LDS), reading P once for the group, and multiplies by the column phasors.
+// Those are products of two table entries, e^{i a(x)} = e^{i a(16 q)}
+// e^{i 2 pi dxy kx r}, x = 16 q + r, so a workgroup's few hundred sincos
+// (double, some 200 instructions) run once, side by side.
+// What bounds it: the latency of that chain at small sizes, the reads of P
+// (from the L2, 16 bytes a point for every group) at large ones.  A round of
+// 39 candidates: 256^2 7.2 -> 6.0 us, 512^2 13.7 -> 9.4, 1024^2 38 -> 19.4
+// against a candidate and four rows per workgroup with a sincos per column;
+// 16 rows 14.6 and 30.1 us at the two larger sizes (too few workgroups); groups of
+// two the same.
+constexpr int kModGroup = 4;
+constexpr int kModRows = 8;
 int modamp_partials_fp64(int nx, int ny) { return (ny + kModRows - 1) / kModRows; }
 
 __device__ __forceinline__ float2 cand_k(const CandSet& s, int c) { return s.kc ? s.kc[c] : s.k[c]; }
-__device__ __forceinline__ int cand_slot(const CandSet& s, int c) { return s.ks ? s.ks[c] : s.slot[c]; }
+__device__ __forceinline__ int cand_slot(const CandSet& s, int c) {
+  return s.nreq ? c / kFitReq : s.ks ? s.ks[c] : s.slot[c];
+}
+// whether candidate c exists (a device-driven fit's round)
+__device__ __forceinline__ bool cand_live(const CandSet& s, int c) {
+  return s.nreq == nullptr || c % kFitReq < s.nreq[c / kFitReq];
+}
 
+// G > 1: blockIdx.y = direction * groups + group of a device-driven fit's
+// round; G = 1: blockIdx.y is the candidate.
+template <int G>
 __global__ __launch_bounds__(256) void k_modamp_fp64(ModampSlots m, CandSet cs, int nx, int ny, float dxy,
                                                      double2* __restrict__ partials) {
-  extern __shared__ double2 alpha[];  // nx phasors
-  __shared__ double2 beta[kModRows];
-  __shared__ double rx[256], ry[256];
-  const int c = blockIdx.y;
-  if (cs.nd != nullptr && c >= *cs.nd) return;  // whole block
-  const double2* __restrict__ P = m.P[cand_slot(cs, c)];
-  const float2 kc = cand_k(cs, c);
-  const double kx = (double)kc.x, ky = (double)kc.y;
+  constexpr int R = kModRows;
+  constexpr int kGroups = (kFitReq + G - 1) / G;
+  extern __shared__ double2 tab[];  // per candidate: R row phasors, 16 fine and nq coarse column phasors
+  __shared__ double red[4][2 * G];
+  int c0 = blockIdx.y, nc = 1;
+  if (G > 1) {
+    const int d = blockIdx.y / kGroups, i0 = (blockIdx.y % kGroups) * G;
+    c0 = d * kFitReq + i0;
+    nc = min(G, cs.nreq[d] - i0);
+    if (nc <= 0) return;  // whole block
+  }
+  const double2* __restrict__ P = m.P[cand_slot(cs, c0)];
   const double twopi_dxy = 2.0 * 3.14159265358979323846 * (double)dxy;
+  const int j0 = blockIdx.x * R;
+  const int nrows = min(R, ny - j0);
+  P += (long long)j0 * nx;
+  const int nq = (nx + 15) / 16, per = R + 16 + nq;
+  for (int e = threadIdx.x; e < nc * per; e += 256) {
+    const int g = e / per, q = e - g * per;
+    const float2 kc = cand_k(cs, c0 + g);
+    const double pos = q < R ? (double)(j0 + q) - 0.5 * ny : q < R + 16 ? (double)(q - R) : 16.0 * (q - R - 16) - 0.5 * nx;
+    double sn, csn;
+    sincos(twopi_dxy * (pos * (q < R ? (double)kc.y : (double)kc.x)), &sn, &csn);
+    tab[e] = make_double2(csn, sn);
+  }
+  __syncthreads();
+  double ar[G], ai[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) ar[g] = ai[g] = 0.0;
   for (int i = threadIdx.x; i < nx; i += 256) {
-    double sn, cs;
-    sincos(twopi_dxy * (((double)i - 0.5 * nx) * kx), &sn, &cs);
-    alpha[i] = make_double2(cs, sn);
-  }
-  const int j0 = blockIdx.x * kModRows;
-  if (threadIdx.x < kModRows) {
-    double sn, cs;
-    sincos(twopi_dxy * (((double)(j0 + threadIdx.x) - 0.5 * ny) * ky), &sn, &cs);
-    beta[threadIdx.x] = make_double2(cs, sn);
-  }
-  __syncthreads();
-  double ar = 0.0, ai = 0.0;
-  const int nrows = min(kModRows, ny - j0);
-  for (int idx = threadIdx.x; idx < nrows * nx; idx += 256) {
-    const int jj = idx / nx, i = idx - jj * nx;
-    const double2 pv = P[(long long)(j0 + jj) * nx + i];
-    const double2 a = alpha[i], b = beta[jj];
-    const double er = a.x * b.x - a.y * b.y, ei = a.x * b.y + a.y * b.x;
-    ar += pv.x * er - pv.y * ei;
-    ai += pv.x * ei + pv.y * er;
-  }
-  rx[threadIdx.x] = ar;
-  ry[threadIdx.x] = ai;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      rx[threadIdx.x] += rx[threadIdx.x + s];
-      ry[threadIdx.x] += ry[threadIdx.x + s];
+    double2 pv[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) pv[r] = P[(long long)(r < nrows ? r : 0) * nx + i];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      if (g < nc) {  // uniform
+        double tr = 0.0, ti = 0.0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const double2 b = r < nrows ? tab[g * per + r] : make_double2(0.0, 0.0);
+          tr += pv[r].x * b.x - pv[r].y * b.y;
+          ti += pv[r].x * b.y + pv[r].y * b.x;
+        }
+        const double2 lo = tab[g * per + R + (i & 15)], hi = tab[g * per + R + 16 + (i >> 4)];
+        const double er = hi.x * lo.x - hi.y * lo.y, ei = hi.x * lo.y + hi.y * lo.x;
+        ar[g] += tr * er - ti * ei;
+        ai[g] += tr * ei + ti * er;
+      }
     }
-    __syncthreads();
   }
-  if (threadIdx.x == 0) partials[(long long)c * gridDim.x + blockIdx.x] = make_double2(rx[0], ry[0]);
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const double x = wave_total(ar[g]), y = wave_total(ai[g]);
+    if (lane == 0) {
+      red[wave][2 * g] = x;
+      red[wave][2 * g + 1] = y;
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < nc) {
+    const int g = threadIdx.x;
+    const double x = (red[0][2 * g] + red[1][2 * g]) + (red[2][2 * g] + red[3][2 * g]);
+    const double y = (red[0][2 * g + 1] + red[1][2 * g + 1]) + (red[2][2 * g + 1] + red[3][2 * g + 1]);
+    partials[(long long)(c0 + g) * gridDim.x + blockIdx.x] = make_double2(x, y);
+  }
 }
 
 static void check_cands(const CandSet& c, int ncand) {
   if (ncand < 1 || (c.kc == nullptr && ncand > kArgCand) || ncand > 65535)
     throw ArgError("modamp: 1..128 candidates per launch (by value), 1..65535 from device arrays");
-  if ((c.kc == nullptr) != (c.ks == nullptr)) throw ArgError("modamp: candidates and slots from the same source");
+  if (c.nreq != nullptr && (c.kc == nullptr || ncand % kFitReq)) throw ArgError("modamp: a round's candidates come by direction");
+  if (c.nreq == nullptr && (c.kc == nullptr) != (c.ks == nullptr)) throw ArgError("modamp: candidates and slots from the same source");
 }
 
 void launch_modamp_fp64(const ModampSlots& m, const CandSet& c, int ncand, int nx, int ny, float dxy,
                         double2* partials, hipStream_t s) {
   check_cands(c, ncand);
-  dim3 grid(modamp_partials_fp64(nx, ny), ncand);
-  hipLaunchKernelGGL(k_modamp_fp64, grid, dim3(256), sizeof(double2) * nx, s, m, c, nx, ny, dxy, partials);
+  const int nb = modamp_partials_fp64(nx, ny);
+  // a device-driven fit's candidates come by direction and share their reads
+  // of P; other batches have few candidates, or few of one slot
+  const int G = c.nreq != nullptr ? kModGroup : 1;
+  const size_t lds = (size_t)G * (kModRows + 16 + (nx + 15) / 16) * sizeof(double2);
+  if (c.nreq != nullptr)
+    hipLaunchKernelGGL(k_modamp_fp64<kModGroup>, dim3(nb, ncand / kFitReq * ((kFitReq + kModGroup - 1) / kModGroup)),
+                       dim3(256), lds, s, m, c, nx, ny, dxy, partials);
+  else
+    hipLaunchKernelGGL(k_modamp_fp64<1>, dim3(nb, ncand), dim3(256), lds, s, m, c, nx, ny, dxy, partials);
   SIMR_LAUNCH_CHECK();
 }
 
 // The result arithmetic of one modamp candidate, in the host's order and
-// precision (one thread: the sums are sequential in block order).
-__global__ __launch_bounds__(256) void k_modamp_finish(int fp32, ModampSlots m, const int* __restrict__ kslot,
-                                                       const double2* __restrict__ part64,
-                                                       const float4* __restrict__ part32, int nparts, int zblocks,
-                                                       float2* __restrict__ amp, float* __restrict__ corr, int stride,
-                                                       int order) {
+// precision.  fp64: one wavefront per candidate, all in one workgroup, which
+// then publishes the fit it completes (pub.out non-null); fp32: one workgroup
+// per candidate (float sums in block order).
+__global__ __launch_bounds__(64 * kMaxDirs) void k_modamp_finish_fp64(ModampSlots m, const int* __restrict__ kslot,
+                                                                      int ncand, const double2* __restrict__ part64,
+                                                                      int nparts, float2* amp, float* corr, int stride,
+                                                                      int order, const FitState* fit, FitPub pub) {
+#pragma clang fp contract(off)
+  const int c = threadIdx.x / 64;
+  if (c < ncand) {
+    const int slot = kslot[c], zb = m.zb[slot];
+    const double* __restrict__ totals = m.totals[slot];
+    part64 += (long long)c * nparts;
+    double xi;
+    const double xr = quad_sum(nparts, [&](int i) { return part64[i]; }, &xi);
+    const double sx = wave_sum(zb, [&](int i) { return totals[i]; });
+    const double sy = wave_sum(zb, [&](int i) { return totals[zb + i]; });
+    if (threadIdx.x % 64 == 0) {
+      amp[slot * stride + order] = make_float2((float)(xr / sx), (float)(xi / sx));
+      corr[slot * stride + order] = (float)sqrt((xr * xr + xi * xi) / (sx * sy));
+    }
+  }
+  if (pub.out != nullptr) {
+    __syncthreads();
+    fit_publish(fit, pub, amp, corr);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_modamp_finish_fp32(const int* __restrict__ kslot,
+                                                            const float4* __restrict__ part32, int nparts,
+                                                            float2* __restrict__ amp, float* __restrict__ corr,
+                                                            int stride, int order) {
 #pragma clang fp contract(off)
   __shared__ double stage[4 * kSeqChunk];
   __shared__ double sums[4];
   const int c = blockIdx.x, slot = kslot[c];
-  const double* __restrict__ totals = m.totals[slot];
-  part64 += (long long)c * nparts;
   part32 += (long long)c * nparts;
-  amp += slot * stride + order;
-  corr += slot * stride + order;
-  if (fp32) {
-    const float v = seq_sum_lanes<float, 4>(nparts, stage, [&](int i, int k) {
-      const float4 q = part32[i];
-      return (double)(k == 0 ? q.x : k == 1 ? q.y : k == 2 ? q.z : q.w);
-    });
-    if (threadIdx.x < 4) sums[threadIdx.x] = v;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    const float xr = (float)sums[0], xi = (float)sums[1], sx = (float)sums[2], sy = (float)sums[3];
-    const float mx = xr / sx, my = xi / sx;
-    *amp = make_float2(mx, my);
-    *corr = sqrtf((xr * xr + xi * xi) / (sx * sy));
-  } else {
-    const double v = seq_sum_lanes<double, 2>(nparts, stage, [&](int i, int k) {
-      return k == 0 ? part64[i].x : part64[i].y;
-    });
-    if (threadIdx.x < 2) sums[threadIdx.x] = v;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    const double xr = sums[0], xi = sums[1], sx = totals[kZsumFinal], sy = totals[kZsumFinal + 1];
-    *amp = make_float2((float)(xr / sx), (float)(xi / sx));
-    *corr = (float)sqrt((xr * xr + xi * xi) / (sx * sy));
-  }
+  const float v = seq_sum_lanes<float, 4>(nparts, stage, [&](int i, int k) {
+    const float4 q = part32[i];
+    return (double)(k == 0 ? q.x : k == 1 ? q.y : k == 2 ? q.z : q.w);
+  });
+  if (threadIdx.x < 4) sums[threadIdx.x] = v;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  const float xr = (float)sums[0], xi = (float)sums[1], sx = (float)sums[2], sy = (float)sums[3];
+  const float mx = xr / sx, my = xi / sx;
+  amp[slot * stride + order] = make_float2(mx, my);
+  corr[slot * stride + order] = sqrtf((xr * xr + xi * xi) / (sx * sy));
+}
+
+__global__ void k_fit_publish(const FitState* fit, FitPub pub, const float2* amps, const float* corr) {
+  fit_publish(fit, pub, amps, corr);
 }
 
 void launch_modamp_finish(bool fp32, const ModampSlots& m, const int* kslot, int ncand, const double2* part64,
-                          const float4* part32, int nparts, int zblocks, float2* amp, float* corr, int stride,
-                          int order, hipStream_t s) {
+                          const float4* part32, int nparts, float2* amp, float* corr, int stride, int order,
+                          const FitState* fit, const FitPub& pub, hipStream_t s) {
   if (ncand < 1) return;
-  hipLaunchKernelGGL(k_modamp_finish, dim3(ncand), dim3(256), 0, s, fp32 ? 1 : 0, m, kslot, part64, part32, nparts,
-                     zblocks, amp, corr, stride, order);
+  if (ncand > kMaxDirs) throw ArgError("modamp finish: 1..8 candidates");
+  if (fp32) {
+    hipLaunchKernelGGL(k_modamp_finish_fp32, dim3(ncand), dim3(256), 0, s, kslot, part32, nparts, amp, corr, stride,
+                       order);
+    if (pub.out != nullptr) hipLaunchKernelGGL(k_fit_publish, dim3(1), dim3(64), 0, s, fit, pub, amp, corr);
+  } else {
+    hipLaunchKernelGGL(k_modamp_finish_fp64, dim3(1), dim3(64 * ncand), 0, s, m, kslot, ncand, part64, nparts, amp,
+                       corr, stride, order, fit, pub);
+  }
   SIMR_LAUNCH_CHECK();
 }
 
 __global__ __launch_bounds__(256) void k_modamp_evals(int fp32, ModampSlots m, CandSet cs,
                                                       const double2* __restrict__ part64,
-                                                      const float4* __restrict__ part32, int nparts, int zblocks,
+                                                      const float4* __restrict__ part32, int nparts,
                                                       double* __restrict__ out, int host_out) {
 #pragma clang fp contract(off)
   __shared__ double stage[4 * kSeqChunk];
   const int c = blockIdx.x;
-  if (cs.nd != nullptr && c >= *cs.nd) return;  // whole block
+  if (!cand_live(cs, c)) return;  // whole block
   out += 4LL * c;
   if (fp32) {
     const float4* pp = part32 + (long long)c * nparts;
@@ -1006,22 +1051,29 @@ __global__ __launch_bounds__(256) void k_modamp_evals(int fp32, ModampSlots m, C
       return (double)(k == 0 ? q.x : k == 1 ? q.y : k == 2 ? q.z : q.w);
     });
     if (threadIdx.x < 4) out[threadIdx.x] = v;
-    if (host_out) __threadfence_system();
-    return;
+  } else {
+    // a wavefront for each of xr, xi, sx, sy
+    const double2* pp = part64 + (long long)c * nparts;
+    const int slot = cand_slot(cs, c), zb = m.zb[slot];
+    const double* totals = m.totals[slot];
+    const int w = threadIdx.x / 64;
+    double v, xi;
+    if (w < 2) {
+      const double xr = quad_sum(nparts, [&](int i) { return pp[i]; }, &xi);
+      v = w == 0 ? xr : xi;
+    } else {
+      v = wave_sum(zb, [&](int i) { return totals[(w == 2 ? 0 : zb) + i]; });
+    }
+    if (threadIdx.x % 64 == 0) out[w] = v;
   }
-  const double2* pp = part64 + (long long)c * nparts;
-  const double v = seq_sum_lanes<double, 2>(nparts, stage, [&](int i, int k) { return k == 0 ? pp[i].x : pp[i].y; });
-  if (threadIdx.x < 2) out[threadIdx.x] = v;
-  if (threadIdx.x == 2 || threadIdx.x == 3)
-    out[threadIdx.x] = m.totals[cand_slot(cs, c)][kZsumFinal + threadIdx.x - 2];
   if (host_out) __threadfence_system();
 }
 
 void launch_modamp_evals(bool fp32, const ModampSlots& m, const CandSet& c, int ncand, const double2* part64,
-                         const float4* part32, int nparts, int zblocks, double* out, bool host_out, hipStream_t s) {
+                         const float4* part32, int nparts, double* out, bool host_out, hipStream_t s) {
   check_cands(c, ncand);
-  hipLaunchKernelGGL(k_modamp_evals, dim3(ncand), dim3(256), 0, s, fp32 ? 1 : 0, m, c, part64, part32, nparts,
-                     zblocks, out, host_out ? 1 : 0);
+  hipLaunchKernelGGL(k_modamp_evals, dim3(ncand), dim3(256), 0, s, fp32 ? 1 : 0, m, c, part64, part32, nparts, out,
+                     host_out ? 1 : 0);
   SIMR_LAUNCH_CHECK();
 }
 
@@ -1084,7 +1136,7 @@ __global__ __launch_bounds__(256) void k_modamp_fp32(ModampSlots m, CandSet cand
 #pragma clang fp contract(off)
   __shared__ float bx[256], by[256], bs[256], bt[256];
   const int c = blockIdx.z;
-  if (cand.nd != nullptr && c >= *cand.nd) return;  // whole block
+  if (!cand_live(cand, c)) return;  // whole block
   const int slot = cand_slot(cand, c);
   const double2* __restrict__ P = m.P[slot];
   const double* __restrict__ SX = m.SX[slot];

@@ -36,7 +36,7 @@ KERNEL_OF_STAGE = {
     "section_sums": "simr::k_section_sums + simr::k_ratios",
     "rows_fwd": "simr::k_rows_fwd<{nx}, unsigned short>",
     "cols_fwd_y": "simr::k_fft2_cols<{ny}, false, ...>",
-    "cols_fwd_z": "simr::k_fft2_cols<{nz}, false, ...>",
+    "cols_fwd_z": "simr::k_zcols<{nz}>",
     "ov_x": "simr::k_overlaps_x<{nx}>",
     "ov_y": "simr::k_fft2_cols<{ny}, true, ...>",
     "ov_zsum": "simr::k_overlaps_zsum<false, false>",
@@ -45,7 +45,7 @@ KERNEL_OF_STAGE = {
     "modamp": "simr::k_modamp_fp64",
     "findk0_peak": "2D FFT + simr::k_argmax_partial + simr::k_fit_begin",
     "filter": "simr::k_filter<...> (every band of the stack)",
-    "asm_z": "simr::k_asm_z_pair<{zdim}, true> + simr::k_asm_z_pair<{zdim}, false>",
+    "asm_z": "simr::k_asm_z_pair<{zdim}, ...> (two launches) or simr::k_asm_z_reg<{zdim}, ...>",
     "asm_y": "simr::k_asm_y<{ydim}, ...>",
     "asm_x": "simr::k_asm_phasors + simr::k_asm_x<{xdim}, ...>",
 }

@@ -336,6 +336,7 @@ Engine::Engine(const simr_params& p, const float* otf, int device) : P(p), L(Lay
   set_flatfield(nullptr, nullptr);
   std::vector<double> zero(L.nz, 0.0);
   SIMR_HIP(hipMemcpyAsync(sdp_, zero.data(), L.nz * 8, hipMemcpyHostToDevice, stream_));
+  partial_.assign(L.ndirs, false);
   k0_.assign(L.ndirs, make_float2(0, 0));
   k0_time0_ = k0_;
   derive();
@@ -403,6 +404,8 @@ void Engine::update_params(const simr_params& p) {
                "parameter change alters the context's buffer layout; create a new context");
   sync();
   refresh_fit();
+  // (the support radius may change: the next readers may look further)
+  for (int d = 0; d < L.ndirs; ++d) complete_bands(d);
   P = p;
   fit_fp32_ = P.fit_fp64 == 0;
   derive();
@@ -591,14 +594,22 @@ void Engine::load_and_rescale(int it) {
   cur_stage_ = stage_begin("rows_fwd", stream_);
   launch_rows_fwd(fp, src, src_u16, bgp, slp, ratio_, apofact_, bands_, stream_);
   stage_end(cur_stage_, stream_);
+  // The y and z transforms of the columns that the overlaps and the filter
+  // read; the others stay as they are until something asks for them
+  // (complete_bands).
+  zcols_ = z_columns();
+  live_x_ = 0;
+  while (live_x_ < L.nxh && !z_column_dead(zcols_, live_x_, 0)) ++live_x_;
   cur_stage_ = stage_begin("cols_fwd_y", stream_);
-  fft_cols(L.ny, bands_, L.nxh, L.nxh, (long long)L.ndirs * L.nbands * L.nz, (long long)L.nxh * L.ny, false,
+  fft_cols(L.ny, bands_, L.nxh, live_x_, (long long)L.ndirs * L.nbands * L.nz, (long long)L.nxh * L.ny, false,
            stream_);
   stage_end(cur_stage_, stream_);
   if (L.nz > 1) {
     cur_stage_ = stage_begin("cols_fwd_z", stream_);
     const long long plane = (long long)L.nxh * L.ny;
-    if (in_list_z(L.nz)) {
+    if (z_in_registers(L.nz)) {
+      launch_zcols(L.nz, bands_, zcols_, L.ndirs * L.nbands, false, stream_);
+    } else if (in_list_z(L.nz)) {
       fft_cols(L.nz, bands_, plane, plane, (long long)L.ndirs * L.nbands, L.H, false, stream_);
     } else {
       // depths without a transform kernel: direct DFT along z (dft_cols),
@@ -617,8 +628,37 @@ void Engine::load_and_rescale(int it) {
     }
     stage_end(cur_stage_, stream_);
   }
+  std::fill(partial_.begin(), partial_.end(), true);
   preprocessed_ = true;
   fitted_ = processed_ = false;
+}
+
+// The columns of the bands that have readers: the overlaps and the filter
+// look at lateral frequencies within rdistcutoff only.
+ZColumns Engine::z_columns() const {
+  const Geo g = geometry();
+  ZColumns c;
+  c.nxh = L.nxh;
+  c.ny = L.ny;
+  c.dkx = g.dkx;
+  c.dky = g.dky;
+  c.rc2 = (float)((double)g.rdistcutoff * (double)g.rdistcutoff * 1.0002);
+  return c;
+}
+
+// Finishes the transforms of direction dir's bands that load_and_rescale left
+// out (columns without readers), for callers that want or replace whole
+// bands.  The 1D transforms commute, so the order in which a column gets them
+// does not matter.  Once the direction is filtered there is nothing to
+// finish: the filter has written zeros there.
+void Engine::complete_bands(int dir) {
+  if (!partial_[dir]) return;
+  partial_[dir] = false;
+  float2* b = bands_ + (size_t)dir * L.nbands * L.H;
+  if (live_x_ < L.nxh)
+    fft_cols(L.ny, b + live_x_, L.nxh, L.nxh - live_x_, (long long)L.nbands * L.nz, (long long)L.nxh * L.ny, false,
+             stream_);
+  if (L.nz > 1 && z_in_registers(L.nz)) launch_zcols(L.nz, b, zcols_, L.nbands, true, stream_);
 }
 
 // ------------------------------------------------------------ geometry
@@ -1476,6 +1516,8 @@ void Engine::filter_dirs(int d0, int d1, const float2* amps) {
   const int st = stage_begin("filter", stream_);
   launch_filter_batch(f, b, stream_);
   stage_end(st, stream_);
+  if (amps == nullptr)  // (a capture: run_graphed says so at every replay)
+    for (int d = d0; d < d1; ++d) partial_[d] = false;
 }
 
 void Engine::filter_dir(int dir) { filter_dirs(dir, dir + 1, nullptr); }
@@ -1506,7 +1548,7 @@ void Engine::assemble() {
     const Geo g = geometry();
     a.dkx = g.dkx;
     a.dky = g.dky;
-    a.rc2_zero = (float)((double)g.rdistcutoff * (double)g.rdistcutoff * 1.0002);
+    a.rc2_zero = z_columns().rc2;
   }
   cur_stage_ = stage_begin("asm_z", stream_);
   launch_asm_z(a, stream_);
@@ -1610,6 +1652,7 @@ void Engine::run_graphed() {
     same_k0 = std::memcmp(&graph_k0_[d], &k0_[d], sizeof(float2)) == 0;
   if (!graph_exec_ || graph_version_ != param_version_ || !same_k0) build_graph();
   SIMR_HIP(hipGraphLaunch(graph_exec_, stream_));
+  std::fill(partial_.begin(), partial_.end(), false);  // filtered
   const size_t na = (size_t)L.ndirs * L.norders;
   SIMR_HIP(hipMemcpyAsync(fit_host_, amps_dev_, na * 8, hipMemcpyDeviceToHost, stream_));
   SIMR_HIP(hipMemcpyAsync((char*)fit_host_ + na * 8, corr_dev_, na * 4, hipMemcpyDeviceToHost, stream_));
@@ -1690,6 +1733,7 @@ void Engine::set_time0_state(const void* host, size_t bytes) {
 
 void Engine::get_band(int dir, int band, float* host) {
   SIMR_REQUIRE(dir >= 0 && dir < L.ndirs && band >= 0 && band < L.nbands, "band index out of range");
+  complete_bands(dir);
   SIMR_HIP(hipMemcpyAsync(host, bands_ + ((size_t)dir * L.nbands + band) * L.H, L.H * 8, hipMemcpyDeviceToHost,
                           stream_));
   sync();
@@ -1697,6 +1741,7 @@ void Engine::get_band(int dir, int band, float* host) {
 
 void Engine::set_band(int dir, int band, const float* host) {
   SIMR_REQUIRE(dir >= 0 && dir < L.ndirs && band >= 0 && band < L.nbands, "band index out of range");
+  complete_bands(dir);  // the direction's other bands
   SIMR_HIP(hipMemcpyAsync(bands_ + ((size_t)dir * L.nbands + band) * L.H, host, L.H * 8, hipMemcpyHostToDevice,
                           stream_));
   sync();

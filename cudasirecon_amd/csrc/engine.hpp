@@ -115,6 +115,8 @@ class Engine {
 
   void derive();
   Geo geometry() const;
+  ZColumns z_columns() const;
+  void complete_bands(int dir);
   int zd_overlaps() const;
   int fit_order2() const;
   OtfTab otf_table(int dir, int order) const;
@@ -167,6 +169,11 @@ class Engine {
   double *sums_ = nullptr, *sdp_ = nullptr;
   float2* bands_ = nullptr;
   float2* otf_ = nullptr;
+  // directions whose columns beyond zcols_ (beyond live_x_ in x) still lack
+  // their y and z transforms (complete_bands)
+  std::vector<bool> partial_;
+  ZColumns zcols_{};
+  int live_x_ = 0;
   std::vector<FitWork> fw_;  // one per direction, in the staging region
   FitWork dbg_;              // overlap dumps (its own region: they write the staging region)
   int nzs_stride_ = 1;       // planes reserved per overlap: 2 zd_max + 1

@@ -7,7 +7,7 @@
 //     v[r] = a[j + r N/R] * w_N^{r k N/(Ns R)},  r = 0..R-1
 //     v    = DFT_R(v)
 //     b[(j/Ns) Ns R + k + q Ns] = v[q]
-// run for the radix sequence of N (8s first, then 4, 2, 5, 3, 7), Ns = product of
+// run for the radix sequence of N (8s first, then 4, 2, 5, 3, 7, 11 .. 31), Ns = product of
 // the radices already applied.  Forward uses w_N = exp(-2 pi i / N), inverse
 // its conjugate; both unnormalised (as cuFFT).
 //
@@ -54,10 +54,11 @@ constexpr Radices make_radices(int N) {
     out.r[out.n++] = 3;
     m /= 3;
   }
-  while (m % 7 == 0) {
-    out.r[out.n++] = 7;
-    m /= 7;
-  }
+  for (int p : {7, 11, 13, 17, 19, 23, 29, 31})
+    while (m % p == 0) {
+      out.r[out.n++] = p;
+      m /= p;
+    }
   if (m != 1) out.n = -1;  // unsupported factor
   return out;
 }
@@ -96,8 +97,15 @@ __device__ __forceinline__ float2 mul_mi(float2 a) {  // a * (-i) forward, a * (
   return INV ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
 }
 
+// The general odd length (primes above 7, compile-time constants), by the
+// symmetric pairs as dft7 below: (R - 1)^2 / 2 complex-by-real products.
 template <int R, bool INV>
-__device__ __forceinline__ void dft(float2* v);
+__device__ __forceinline__ void dft_odd(float2* v);
+template <int R, bool INV>
+__device__ __forceinline__ void dft(float2* v) {
+  static_assert(R % 2 == 1 && R > 7, "the small radices have their own butterflies");
+  dft_odd<R, INV>(v);
+}
 
 template <>
 __device__ __forceinline__ void dft<1, false>(float2*) {}

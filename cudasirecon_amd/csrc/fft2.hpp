@@ -73,6 +73,58 @@ constexpr CS unit(long long m, long long n) {
 }
 }  // namespace ctrig
 
+// cos and sin of 2 pi m / R, m < R, as compile-time floats
+template <int R>
+struct COdd {
+  float c[R], s[R];
+  constexpr COdd() : c{}, s{} {
+    for (int m = 0; m < R; ++m) {
+      c[m] = (float)ctrig::unit(m, R).c;
+      s[m] = (float)ctrig::unit(m, R).s;
+    }
+  }
+};
+template <int R, int M, int K>
+__device__ __forceinline__ void odd_terms(const float2* t, const float2* u, float2& a, float2& b) {
+  if constexpr (K <= (R - 1) / 2) {
+    constexpr COdd<R> w;
+    constexpr float c = w.c[(M * K) % R], s = w.s[(M * K) % R];
+    a.x += c * t[K].x;
+    a.y += c * t[K].y;
+    b.x += s * u[K].x;
+    b.y += s * u[K].y;
+    odd_terms<R, M, K + 1>(t, u, a, b);
+  }
+}
+template <int R, bool INV, int M>
+__device__ __forceinline__ void odd_outputs(float2* v, const float2* t, const float2* u) {
+  if constexpr (M <= (R - 1) / 2) {
+    float2 a = t[0], b = make_float2(0.f, 0.f);
+    odd_terms<R, M, 1>(t, u, a, b);
+    // X_M = a - i b, X_{R-M} = a + i b (forward)
+    const float2 m = make_float2(a.x + b.y, a.y - b.x), q = make_float2(a.x - b.y, a.y + b.x);
+    v[M] = INV ? q : m;
+    v[R - M] = INV ? m : q;
+    odd_outputs<R, INV, M + 1>(v, t, u);
+  }
+}
+template <int R, bool INV>
+__device__ __forceinline__ void dft_odd(float2* v) {
+  constexpr int H = (R - 1) / 2;
+  float2 t[H + 1], u[H + 1];
+  t[0] = v[0];
+  u[0] = make_float2(0.f, 0.f);
+  float2 sum = v[0];
+#pragma unroll
+  for (int k = 1; k <= H; ++k) {
+    t[k] = cadd(v[k], v[R - k]);
+    u[k] = csub(v[k], v[R - k]);
+    sum = cadd(sum, t[k]);
+  }
+  v[0] = sum;
+  odd_outputs<R, INV, 1>(v, t, u);
+}
+
 // exp(-2 pi i m / n) (forward) or its conjugate, as compile-time floats
 template <long long M, long long NN, bool INV>
 struct CTw {
@@ -163,7 +215,7 @@ __device__ __forceinline__ void reg_gather(float2* o, const float2* v) {
 template <int M, bool INV>
 __device__ __forceinline__ void reg_dft(float2* v) {
   if constexpr (M > 1) {
-    static_assert(make_radices(M).n > 0, "register DFT length must factor into 2, 3, 5");
+    static_assert(make_radices(M).n > 0, "register DFT length must factor into primes up to 31");
     dif_stages<M, INV, 0>(v);
     float2 o[M];
     reg_gather<M>(o, v);

@@ -35,7 +35,7 @@ constexpr int rp_dft_cost(int n) {
   const Radices rd = make_radices(n);
   if (rd.n < 0) return 1000;
   int c = 0;
-  for (int i = 0; i < rd.n; ++i) c += rd.r[i] == 8 ? 8 : rd.r[i] == 4 ? 4 : rd.r[i] == 2 ? 2 : rd.r[i] == 3 ? 5 : rd.r[i] == 5 ? 8 : 12;
+  for (int i = 0; i < rd.n; ++i) c += rd.r[i] == 8 ? 8 : rd.r[i] == 4 ? 4 : rd.r[i] == 2 ? 2 : rd.r[i] == 3 ? 5 : rd.r[i] == 5 ? 8 : 5 + rd.r[i];
   return c + 3 * (rd.n - 1);
 }
 constexpr int rp_pow2(int n) {

@@ -312,6 +312,22 @@ struct FilterBatch {
 };
 void launch_filter_batch(const FilterParams& p, const FilterBatch& b, hipStream_t s);
 
+// ---- z transforms in registers ------------------------------------------------
+// Lateral columns (x < nxh, ky row < ny) and the square of the support radius
+// outside which no reader of the bands looks (with a margin; 1/um^2).
+struct ZColumns {
+  int nxh, ny;
+  float dkx, dky, rc2;
+};
+__host__ __device__ inline bool z_column_dead(const ZColumns& c, int x, int row) {
+  const float kx = (float)x * c.dkx, ky = (float)(2 * row > c.ny ? row - c.ny : row) * c.dky;
+  return kx * kx + ky * ky > c.rc2;
+}
+bool z_in_registers(int n);
+// The forward z transforms of n planes, in place, of the columns inside the
+// support (dead: of the others) of `volumes` volumes [n][ny][nxh].
+void launch_zcols(int n, float2* data, const ZColumns& c, int volumes, bool dead, hipStream_t s);
+
 // ---- assembly ----------------------------------------------------------------
 struct AsmParams {
   int nx, ny, nz, nxh;
@@ -331,6 +347,14 @@ struct AsmParams {
   // a margin (0: unknown, nothing is skipped)
   float dkx, dky, rc2_zero;
 };
+// Whether centred column (x, y) lies beyond the filter's support of squared
+// radius rc2 (y above ny/2: the frequency y - ny).
+__device__ __forceinline__ bool asm_dead(const AsmParams& p, int x, int y, float rc2) {
+  const float kx = (float)x * p.dkx, ky = (float)(2 * y > p.ny ? y - p.ny : y) * p.dky;
+  return rc2 > 0.f && kx * kx + ky * ky > rc2;
+}
+bool asm_z_in_registers(const AsmParams& p);
+void launch_asm_z_reg(const AsmParams& p, hipStream_t s);
 // Requests the twiddle tables of the y and x passes (nx, ny, xdim, ydim are
 // read), so that their launches do not allocate.
 void asm_y_request_tables(const AsmParams& p);

@@ -349,8 +349,6 @@ __global__ __launch_bounds__((AsmY<N, HALVES>::NT), (AsmY<N, HALVES>::WAVES)) vo
   // Rows beyond the filter's support in this column are zero; the z pass
   // does not write them.  The bound is taken a little inside the z pass's
   // (rc2_zero), so rounding never reads an element that was not written.
-  const float kx = (float)(xc - (p.nx / 2 - 1)) * p.dkx;
-  const float ymax2 = p.rc2_zero > 0.f ? (p.rc2_zero * 0.9999f - kx * kx) : 3.4e38f;
   const int hy = p.ny / 2 - 1;
   float2 in[K::R1 * N1];
 #pragma unroll
@@ -369,8 +367,7 @@ __global__ __launch_bounds__((AsmY<N, HALVES>::NT), (AsmY<N, HALVES>::WAVES)) vo
         y = lo ? n : n - N;
         live = lo || hi;
       }
-      const float ky = (float)y * p.dky;
-      live = live && ky * ky <= ymax2;
+      live = live && !asm_dead(p, xc - (p.nx / 2 - 1), y, p.rc2_zero * 0.9999f);
       const float2 t = src[(long long)(live ? y + hy : hy) * p.nx];
       in[c * N1 + n1] = live ? t : make_float2(0.f, 0.f);
     }
@@ -463,6 +460,10 @@ static void launch_asm_z_any(const AsmParams& p, hipStream_t s) {
 }
 
 void launch_asm_z(const AsmParams& p, hipStream_t s) {
+  if (asm_z_in_registers(p)) {
+    launch_asm_z_reg(p, s);
+    return;
+  }
   switch (p.zdim) {
 #define SIMR_CASE(N)                                                                              \
   case N: {                                                                                       \

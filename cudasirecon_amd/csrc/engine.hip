@@ -764,6 +764,7 @@ void Engine::make_overlaps(const std::vector<OvReq>& reqs, bool per_elem, FitWor
     z.SY[k] = w.SY;
     z.totals[k] = w.sumparts;
     z.cc[k] = want_cc ? w.cc : nullptr;
+    z.sup[k] = ov_support(b.p[k]);
     z.nzs[k] = 2 * b.p[k].zd + 1;
     w.zd = b.p[k].zd;
     w.cache.clear();

@@ -5,7 +5,8 @@
 //
 //   X[k1 + N1 k2] = sum_{n2} W_N2^{n2 k2} W_N^{n2 k1} sum_{n1} W_N1^{n1 k1} x[N2 n1 + n2]
 //
-// T lanes (a power of two >= the rows of the intermediate) work on one
+// T lanes (at least the rows of the intermediate; a power of two unless the
+// plan's RpWant says otherwise) work on one
 // transform: pass 1, lane j takes columns n2 = j, j + T, ...; pass 2, lane j
 // takes row j and ends with X[j + rows k2].
 //
@@ -48,7 +49,15 @@ constexpr int rp_pow2(int n) {
 // the two halves of a 2M-point one, else 1.  Lane-instructions per output
 // decide; more than 40 values per lane cost occupancy and are taken only
 // where nothing else divides the length.
-constexpr RpPlan rp_plan(int len, int halves) {
+// RpWant bounds the values a lane holds in each pass (kernels with a short
+// chain per thread, or with other registers to keep; taken only if a split
+// within the bounds exists, else rp_plan is empty), and lets T be any multiple
+// of 4 where the lanes of a transform need not share a wavefront.
+struct RpWant {
+  int max1 = 100, max2 = 80;
+  bool any_t = false;
+};
+constexpr RpPlan rp_plan(int len, int halves, RpWant want = RpWant()) {
   RpPlan best{0, 0, 0, 0};
   long long best_cost = 0;
   for (int n1 = 2; n1 <= 64; ++n1) {
@@ -58,9 +67,9 @@ constexpr RpPlan rp_plan(int len, int halves) {
     for (int hl = 1; hl <= halves; ++hl) {
       const int rows = hl * n1;
       if (rows > 64) continue;
-      const int t = rp_pow2(rows);
+      const int t = want.any_t ? (rows + 3) / 4 * 4 : rp_pow2(rows);
       const int r1 = (n2 + t - 1) / t;
-      if (r1 * hl * n1 > 100) continue;
+      if (r1 * hl * n1 > want.max1 || n2 > want.max2) continue;
       // per value: input loads (6), twiddle and exchange (7); the odd half's ramp
       long long c = (long long)r1 * n1 * (hl * (rp_dft_cost(n1) + 7) + 6);
       if (halves == 2) c += (hl == 2 ? 4 : 2) * r1 * n1;
@@ -76,12 +85,20 @@ constexpr RpPlan rp_plan(int len, int halves) {
   }
   return best;
 }
-constexpr bool rp_ok(int len, int halves) { return rp_plan(len, halves).n1 > 0; }
+constexpr bool rp_ok(int len, int halves, RpWant want = RpWant()) { return rp_plan(len, halves, want).n1 > 0; }
 
 // HALVES as in rp_plan; NT2 = HALVES * LEN is the length of the twiddle table.
-template <int LEN, int HALVES>
+// WANT: the index of the kernel's RpWant in kRpWants.
+constexpr RpWant kRpWants[] = {
+    RpWant(),
+    RpWant{24, 24, true},   // 1: short columns of workgroup-wide tiles
+    RpWant{32, 32, true},   // 2: the same, longer columns
+    RpWant{32, 20, false},  // 3: rows whose products are summed in doubles beside them
+    RpWant{32, 32, false},  // 4: the same, longer rows
+};
+template <int LEN, int HALVES, int WANT = 0>
 struct Rp {
-  static constexpr RpPlan P = rp_plan(LEN, HALVES);
+  static constexpr RpPlan P = rp_plan(LEN, HALVES, kRpWants[WANT]);
   static_assert(P.n1 > 0, "no plan for this length");
   static constexpr int N1 = P.n1, N2 = P.n2, HL = P.hl, T = P.lanes;
   static constexpr int ROWS = HL * N1;                  // rows of one transform's intermediate
@@ -128,11 +145,11 @@ __device__ __forceinline__ void rp_sync() {
 // j >= ROWS: nothing useful).  buf is free again after the caller's next
 // rp_sync.  WAVE: the T lanes lie in one wavefront and no other touches buf;
 // otherwise workgroup barriers, and every thread of the workgroup calls it.
-template <int LEN, int HALVES, bool INV, bool WAVE>
+template <int LEN, int HALVES, bool INV, bool WAVE, int WANT = 0>
 __device__ __forceinline__ void rp_transform(float* buf, int j, bool odd, const float2* tw,
-                                             const float2 (&in)[Rp<LEN, HALVES>::R1 * Rp<LEN, HALVES>::N1],
-                                             float2 (&out)[Rp<LEN, HALVES>::N2]) {
-  using K = Rp<LEN, HALVES>;
+                                             const float2 (&in)[Rp<LEN, HALVES, WANT>::R1 * Rp<LEN, HALVES, WANT>::N1],
+                                             float2 (&out)[Rp<LEN, HALVES, WANT>::N2]) {
+  using K = Rp<LEN, HALVES, WANT>;
   constexpr int N1 = K::N1, N2 = K::N2, HL = K::HL, R1 = K::R1;
   float2 v[R1 * HL * N1];
 #pragma unroll

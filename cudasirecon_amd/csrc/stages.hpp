@@ -74,6 +74,14 @@ struct OvParams {
   const float2* k0d;
   float kmul;
 };
+// What decides which elements of an overlap pair can differ from zero.
+struct OvSupport {
+  float kx, ky;         // OvParams'
+  const float2* k0d;
+  float kmul;
+  float rc2, dkx, dky;
+  int nx, ny, zd, bNoKz0;
+};
 struct OvBatch {
   OvParams p[kMaxDirs];
   int n;           // slots
@@ -103,6 +111,8 @@ struct ZsumBatch {
   // non-null: also conj(P) in float there (the cross-correlation's input:
   // aTimesConjB, X conj(Y) = conj(conj(X) Y))
   float2* cc[kMaxDirs];
+  // the two-pass form: what the column pass left out (OvParams' support)
+  OvSupport sup[kMaxDirs];
   int nzs[kMaxDirs];
   int n, nzs_stride, nz;
   long long nxy;
@@ -113,6 +123,7 @@ void launch_overlaps_z_reduce(const ZsumBatch& b, bool fp32, bool per_elem, hipS
 // inverse x transform with the z sums (by rows, ..._rows); P and the totals
 // as launch_overlaps_z_reduce(fp32 = false, per_elem = false) leaves them.
 // overlaps_fused_ok: whether the geometry is covered.
+OvSupport ov_support(const OvParams& p);
 bool overlaps_fused_ok(const OvBatch& ob, const ZsumBatch& zb);
 void launch_overlaps_fused_cols(const OvBatch& ob, hipStream_t s);
 void launch_overlaps_fused_rows(const ZsumBatch& zb, int nx, int ny, hipStream_t s);

@@ -24,6 +24,7 @@
 #include "fft.hpp"
 #include "fft2.hpp"
 #include "fft_api.hpp"
+#include "fft_rp.hpp"
 #include "fit_device.hpp"
 #include "sizes.hpp"
 #include "stages.hpp"
@@ -350,49 +351,92 @@ void launch_overlaps_x(const OvBatch& b, hipStream_t s) {
 // than the three-pass form's, so P agrees with it to rounding, not bit for
 // bit.
 
-// Whether column j of overlap `which` can hold a nonzero element (the row
-// test of ov_row_live with x and y exchanged).
-__device__ __forceinline__ bool ov_col_live(const OvParams& p, float kx, float ky, int which, int j, int z0) {
-  if (j >= p.nx || (z0 == 0 && p.bNoKz0)) return false;
-  float x = (float)j;
-  if (x > (float)(p.nx / 2)) x -= (float)p.nx;
-  x *= p.dkx;
-  const float sx = which == 0 ? kx : -kx, sy = which == 0 ? ky : -ky;
-  const float r2 = p.rc2 * 1.0002f;
-  const float a2 = r2 - x * x, b2 = r2 - (x - sx) * (x - sx);
-  if (a2 < 0.f || b2 < 0.f) return false;
-  return fabsf(sy) <= (sqrtf(a2) + sqrtf(b2)) * 1.0001f;
+OvSupport ov_support(const OvParams& p) {
+  return OvSupport{p.kx, p.ky, p.k0d, p.kmul, p.rc2, p.dkx, p.dky, p.nx, p.ny, p.zd, p.bNoKz0};
+}
+__device__ __forceinline__ float2 ov_shift(const OvSupport& q) {
+#pragma clang fp contract(off)
+  if (q.k0d == nullptr) return make_float2(q.kx, q.ky);
+  const float2 k = *q.k0d;
+  return make_float2(k.x * q.kmul, k.y * q.kmul);
 }
 
-// columns per workgroup of the column pass (radix-stage core: its rows are
-// a quarter of the two-pass core's LDS per thread, which keeps the occupancy
-// the formation's gathers need)
-template <int NY>
-constexpr int ovf_cols_w() {
-  int w = 8;
-  while (w > 1 && w * fft_tpt(NY) > 512) w /= 2;
-  return w;
+// The range of centred columns of overlap `which` (shift k) that can hold a
+// nonzero element: those whose frequency lies in the x extent of the lens
+// |q| <= rc, |q - s| <= rc (s = k, or -k for overlap1).  Its rightmost point is
+// one disc's, if that lies in the other disc, else the discs' right
+// intersection; likewise on the left.  The range carries a margin far beyond
+// the rounding of the per-element tests; hi < lo: no column.  (Plane kz = 0
+// with bNoKz0 is left to the callers.)
+__device__ __forceinline__ float2 ov_col_range(const OvSupport& p, float2 k, int which) {
+  const float sx = which == 0 ? k.x : -k.x, sy = which == 0 ? k.y : -k.y;
+  const float r2 = p.rc2 * 1.0002f, r = __builtin_amdgcn_sqrtf(r2);
+  const float d2 = sx * sx + sy * sy;
+  if (d2 > 4.f * r2) return make_float2(1.f, 0.f);
+  // half the chord through the intersections, along x
+  const float h = __builtin_amdgcn_sqrtf(fmaxf(r2 - 0.25f * d2, 0.f));
+  const float chord = d2 > 0.f ? fabsf(sy) * h * __builtin_amdgcn_rsqf(d2) : r;
+  // the right end of the disc further left, if inside the other; else the intersection
+  const float e2 = (r - fabsf(sx)) * (r - fabsf(sx)) + sy * sy;  // its squared distance from the other's centre
+  const float half = e2 <= r2 ? r - 0.5f * fabsf(sx) : chord;    // the lens is symmetric about s / 2
+  const float m = 1e-3f * r;
+  return make_float2(0.5f * sx - half - m, 0.5f * sx + half + m);
 }
+__device__ __forceinline__ bool ov_col_live(const OvSupport& p, float2 range, int j) {
+  const float x = (float)(j > p.nx / 2 ? j - p.nx : j) * p.dkx;
+  return x >= range.x && x <= range.y;
+}
+
+// The column pass: W adjacent columns of overlap blockIdx.x % 2 on plane
+// blockIdx.y of slot blockIdx.z.  Thread (w, j) forms its pass-1 inputs of
+// column c0 + w (as k_overlaps_x) straight in registers, transforms them on the
+// two-pass register core and stores its outputs; LDS holds one float per
+// element.  Tiles without a live column are left unwritten, and the row pass
+// does not read them.
+// What bounds it is the formation (two radial lookups, square roots and a
+// normalisation per element) and its chain of dependent loads, so the plans ask
+// for few values a lane (24, else 32) and many wavefronts.  On the radix stages in LDS, every element a trip
+// through LDS per stage and dead tiles filled with zeros: 175.6 us in
+// a 512x512x48 stack (a launch is three directions), 350 in 1024x1024x16,
+// 29.0 in 256x256x32 and 11.2 in one 256x256 plane; now 149, 206, 26.0 and 12.6
+// (that one is latency: the shift, the profile, the bands, the twiddles).
+// 480x400x21 and 384x384x26, at three passes before: the row pass's figures.
+template <int NY>
+constexpr int ovc_want() {
+  return rp_ok(NY, 1, kRpWants[1]) ? 1 : rp_ok(NY, 1, kRpWants[2]) ? 2 : 0;
+}
+template <int NY>
+struct OvC {
+  static constexpr int WANT = ovc_want<NY>();
+  using K = Rp<NY, 1, WANT>;
+  static constexpr int span_of(int w) {  // columns offset by 32 / w banks
+    const int want = w < 32 ? 32 / w : 1;
+    return K::SPAN + ((want - K::SPAN % 32) % 32 + 32) % 32;
+  }
+  static constexpr int width() {
+    int w = NY <= 256 ? 8 : 16;  // (small planes: more workgroups)
+    while (w > 4 && (w * K::T > 512 || w * span_of(w) * 4 > 72 * 1024)) w /= 2;
+    while (w * K::T % 64) w *= 2;  // whole wavefronts
+    return w;
+  }
+  static constexpr int W = width(), NT = W * K::T;
+  static constexpr int LDS = W * span_of(W) * 4;
+  static constexpr int VALUES = K::R1 * K::N1 > K::N2 ? K::R1 * K::N1 : K::N2;
+  // (128 VGPRs at four wavefronts per SIMD; factors of 5 spill there)
+  static constexpr int WAVES = VALUES <= 32 ? (NY % 25 == 0 ? 3 : 4) : VALUES <= 40 ? 2 : 1;
+};
 template <int NY>
 constexpr bool ovf_cols_ok() {
-  return fft_supported(NY) && NY > 1 && (ovf_cols_w<NY>() * lds_pitch(NY) + NY) * 8 <= 64 * 1024 &&
-         (NY * ovf_cols_w<NY>()) % (ovf_cols_w<NY>() * fft_tpt(NY)) == 0;
+  return OvC<NY>::NT <= 1024 && OvC<NY>::LDS <= 128 * 1024;
 }
 
-// Columns [W*(blockIdx.x/2), +W) of overlap blockIdx.x%2 on plane blockIdx.y
-// of slot blockIdx.z: formation (as k_overlaps_x) and the inverse y transform.
 template <int NY, bool RA>
-__global__ __launch_bounds__(ovf_cols_w<NY>() * fft_tpt(NY)) void k_ovf_cols(OvBatch b,
-                                                                          const float2* __restrict__ tw) {
-  constexpr int W = ovf_cols_w<NY>();
-  constexpr int TPT = fft_tpt(NY);
-  constexpr int NT = W * TPT;
-  constexpr int P = lds_pitch(NY);
-  constexpr int EPT = NY * W / NT;
-  constexpr int CH = EPT < 4 ? EPT : 4;
-  static_assert(EPT % CH == 0, "chunks cover the elements");
-  // XCD-contiguous tile order: neighbouring column tiles, whose 64-byte
-  // segments of the 257-element band rows share cache lines, run in one L2
+__global__ __launch_bounds__(OvC<NY>::NT, OvC<NY>::WAVES) void k_ovf_cols(OvBatch b, const float2* __restrict__ tw) {
+  using C = OvC<NY>;
+  using K = typename C::K;
+  constexpr int W = C::W, NT = C::NT, N1 = K::N1, N2 = K::N2;
+  // XCD-contiguous tile order: neighbouring column tiles, whose segments of
+  // the nx/2+1-element band rows share cache lines, run in one L2
   unsigned bx, by, bz;
   xcd_tile3(bx, by, bz);
   const OvParams& p = b.p[bz];
@@ -401,48 +445,41 @@ __global__ __launch_bounds__(ovf_cols_w<NY>() * fft_tpt(NY)) void k_ovf_cols(OvB
   const int which = bx & 1;
   const int c0 = (bx >> 1) * W;
   const int z0 = zb - p.zd;
-  float kx = p.kx, ky = p.ky;
-  if (p.k0d != nullptr) {
-#pragma clang fp contract(off)
-    const float2 k = *p.k0d;
-    kx = k.x * p.kmul;
-    ky = k.y * p.kmul;
-  }
-  float2* __restrict__ plane = p.ovx + ((long long)which * b.nzs_stride + zb) * NY * p.nx;
+  if (z0 == 0 && p.bNoKz0) return;
+  const OvSupport sup{p.kx, p.ky, p.k0d, p.kmul, p.rc2, p.dkx, p.dky, p.nx, p.ny, p.zd, p.bNoKz0};
+  const float2 k = ov_shift(sup);
   {
+    const float2 range = ov_col_range(sup, k, which);
     bool live = false;
-    for (int w = 0; w < W; ++w) live = live || ov_col_live(p, kx, ky, which, c0 + w, z0);
-    if (!live) {
-      for (int idx = threadIdx.x; idx < NY * W; idx += NT) {
-        const int i = idx / W, w = idx % W;
-        if (c0 + w < p.nx) plane[(long long)i * p.nx + c0 + w] = make_float2(0.f, 0.f);
-      }
-      return;  // uniform over the workgroup
-    }
+    for (int w = 0; w < W; ++w) live = live || (c0 + w < p.nx && ov_col_live(sup, range, c0 + w));
+    if (!live) return;  // uniform over the workgroup
   }
-  __shared__ float2 lds[W * P];
+  __shared__ float buf[C::LDS / 4];
   extern __shared__ float2 prof[];  // [2][nxotf]
-  const int tid = threadIdx.x;
-  FftTw<NY> twr;
-  __shared__ float2 twstage[NY];
-  load_twiddles(twr, twstage, tid % TPT, tw, tid, NT);
+  const int w = threadIdx.x % W, j = threadIdx.x / W;
   const int nxotf = p.otf1.nxotf;
-  if constexpr (RA)
-    for (int k = tid; k < 2 * nxotf; k += NT)
-      prof[k] = otf_profile_entry(k < nxotf ? p.otf1 : p.otf2, k < nxotf ? k : k - nxotf, z0, p.kzscale);
-  __syncthreads();
+  if constexpr (RA) {
+    for (int i = threadIdx.x; i < 2 * nxotf; i += NT)
+      prof[i] = otf_profile_entry(i < nxotf ? p.otf1 : p.otf2, i < nxotf ? i : i - nxotf, z0, p.kzscale);
+    __syncthreads();
+  }
+  const int jc = c0 + w < p.nx ? c0 + w : p.nx - 1;
   const float2* bre = which == 0 ? p.b1re : p.b2re;
   const float2* bim = which == 0 ? (p.order1 > 0 ? p.b1im : p.b1re) : p.b2im;
   const bool has_im = which == 1 || p.order1 > 0;
+  float2 in[K::R1 * N1];
+  // in chunks: the sources of a chunk first, then all its band loads (clamped
+  // to a valid index for zero elements), then the products
+  constexpr int E = K::R1 * N1, CH = E <= 16 ? (E < 8 ? E : 8) : 4;
 #pragma unroll
-  for (int q0 = 0; q0 < EPT; q0 += CH) {
+  for (int q0 = 0; q0 < E; q0 += CH) {
     OvSrc src[CH];
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      const int idx = tid + (q0 + c) * NT;
-      const int i = idx / W, j = c0 + idx % W;
-      src[c] = j < p.nx ? ov_source<RA>(p, kx, ky, prof, prof + nxotf, which, j, i, z0)
-                        : OvSrc{0, false, false, make_float2(0.f, 0.f)};
+      const int e = q0 + c < E ? q0 + c : E - 1;
+      const int n2 = j + K::T * (e / N1);
+      const int i = N2 * (e % N1) + (K::N2 % K::T == 0 || n2 < N2 ? n2 : N2 - 1);
+      src[c] = ov_source<RA>(p, k.x, k.y, prof, prof + nxotf, which, jc, i, z0);
     }
     float2 vre[CH], vim[CH];
 #pragma unroll
@@ -451,128 +488,205 @@ __global__ __launch_bounds__(ovf_cols_w<NY>() * fft_tpt(NY)) void k_ovf_cols(OvB
       vim[c] = bim[src[c].ind];
     }
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int idx = tid + (q0 + c) * NT;
-      lds[(idx % W) * P + lds_swz<NY>(idx / W)] = ov_combine(src[c], vre[c], vim[c], has_im);
-    }
+    for (int c = 0; c < CH; ++c)
+      if (q0 + c < E) in[q0 + c] = ov_combine(src[c], vre[c], vim[c], has_im);
   }
-  __syncthreads();
-  fft_lds<NY, true>(lds + (tid / TPT) * P, tid % TPT, twr);
+  float2 out[N2];
+  rp_transform<NY, 1, true, false, C::WANT>(buf + w * C::span_of(W), j, false, tw, in, out);
+  if (c0 + w < p.nx && (K::ROWS == K::T || j < K::ROWS)) {
+    float2* col = p.ovx + (((long long)which * b.nzs_stride + zb) * NY + j) * p.nx + c0 + w;
 #pragma unroll
-  for (int k = 0; k < EPT; ++k) {
-    const int idx = tid + k * NT;
-    const int i = idx / W, w = idx % W;
-    if (c0 + w < p.nx) plane[(long long)i * p.nx + c0 + w] = lds[w * P + lds_swz<NY>(i)];
+    for (int k2 = 0; k2 < N2; ++k2) col[(long long)(K::OSTEP * k2) * p.nx] = out[k2];
   }
 }
 
-// planes per round of the row pass: G of each overlap, 2G transforms on the
-// radix-stage core
-constexpr int kOvfG = 4;
+// The row pass.  Two groups of T lanes take a plane of row y, one transforming
+// X and the other Y on the two-pass register core (wave-private exchange); the
+// groups then swap halves of their outputs (lane swaps in registers), so each
+// holds X and Y of half the row and adds the products up in its registers, plane
+// after plane.  The pairs' sums meet in LDS at the end.
+// What bounds it is latency at two to four wavefronts a SIMD: the double sums
+// and a row's values fill the registers, so a lane holds half the sums, and
+// plans of at most 32 values.  (One group transforming X, then Y, with all the
+// sums, spilled at every length above 80.)  Four wavefronts to a workgroup: the
+// wavefronts of a SIMD come from several rows.  Live columns only are read.
+// Per launch, three directions: 1024x1024x16 224.5 us before (radix stages in
+// LDS) and 160 now; 512x512x48 96.9 and 104.5, which the column pass wins back
+// (272.5 the pair, now 254).  Sizes that had three passes, both kernels:
+// 480x400x21 164.5, now 108; 384x384x26 144.4, now 125; 64x64x9 24.2, now 16.
+template <int NX>
+constexpr int ovr_want() {
+  return NX < 300 && rp_ok(NX, 1, kRpWants[3]) ? 3 : 4;
+}
+template <int NX>
+struct OvR {
+  static constexpr int WANT = ovr_want<NX>();
+  using K = Rp<NX, 1, WANT>;
+  static constexpr int HALF = (K::N2 + 1) / 2;  // outputs a lane accumulates
+  static constexpr int SPANP = K::SPAN + ((K::T - K::SPAN % 32) % 32 + 32) % 32;
+  static constexpr int MAXP = 256 / (2 * K::T) < 8 ? 256 / (2 * K::T) : 8;  // pairs per workgroup
+  static constexpr int threads(int pairs) { return (pairs * 2 * K::T + 63) / 64 * 64; }
+  // twiddles; then the exchange buffers, which the pairs' sums reuse
+  static constexpr int lds(int pairs) {
+    const int ex = threads(pairs) / K::T * SPANP * 4, sums = (pairs + 1) / 2 * NX * 16;
+    return K::TABN * 8 + (ex > sums ? ex : sums);
+  }
+  static constexpr int WAVES = K::N2 > 16 || K::R1 * K::N1 > 24 ? 2 : 3;
+  static_assert(K::TABN % 2 == 0, "the double2 sums are 16-byte aligned");
+};
 template <int NX>
 constexpr bool ovf_rows_ok() {
-  return fft_supported(NX) && NX > 1 && 2 * kOvfG * fft_tpt(NX) <= 1024 && 2 * kOvfG * fft_tpt(NX) >= 64 &&
-         (2 * kOvfG * lds_pitch(NX) + NX) * 8 <= 96 * 1024 && (2 * kOvfG * NX) % (2 * kOvfG * fft_tpt(NX)) == 0;
+  if constexpr (rp_ok(NX, 1, kRpWants[ovr_want<NX>()]))
+    return OvR<NX>::K::T <= 32 && OvR<NX>::lds(OvR<NX>::MAXP) <= 150 * 1024;
+  return false;
 }
 
-// Row y = blockIdx.x of every stored plane of both overlaps of slot
-// blockIdx.y: the inverse x transforms, kOvfG planes at a time, then
-// P(x, y) = nz sum_kz conj(X) Y in plane order (as k_overlaps_zsum), and the
-// block's share of the SX and SY totals.
+// a of the odd group of T lanes <-> b of the even group next to it
+template <int T>
+__device__ __forceinline__ void ov_swap(float& a, float& b) {
+  if constexpr (T == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  } else if constexpr (T == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  } else {
+    const bool odd = threadIdx.x & T;
+    const float got = __shfl_xor(odd ? a : b, T);
+    if (odd)
+      a = got;
+    else
+      b = got;
+  }
+}
+
 template <int NX>
-__global__ __launch_bounds__(2 * kOvfG * fft_tpt(NX)) void k_ovf_rows(ZsumBatch b, const float2* __restrict__ tw) {
+__global__ __launch_bounds__(OvR<NX>::threads(OvR<NX>::MAXP), OvR<NX>::WAVES) void k_ovf_rows(
+    ZsumBatch b, int pairs, const float2* __restrict__ tw) {
 #pragma clang fp contract(off)
-  constexpr int TPT = fft_tpt(NX);
-  constexpr int NT = 2 * kOvfG * TPT;
-  constexpr int P = lds_pitch(NX);
-  constexpr int EPT = (NX + NT - 1) / NT;  // output elements per thread
-  constexpr int LPT = 2 * kOvfG * NX / NT;  // loads per thread per round
-  __shared__ float2 lds[2 * kOvfG * P];
-  __shared__ double red[NT];
-  const int tid = threadIdx.x;
+  using C = OvR<NX>;
+  using K = typename C::K;
+  constexpr int T = K::T, N1 = K::N1, N2 = K::N2, HALF = C::HALF;
+  extern __shared__ float2 twl[];
+  __shared__ double red[2][16];
   const int y = blockIdx.x, slot = blockIdx.y;
+  const OvSupport& sup = b.sup[slot];
+  const float2 k = ov_shift(sup);  // (in flight with the twiddles)
+  for (int i = threadIdx.x; i < K::TABN; i += blockDim.x) twl[i] = tw[i];
+  __syncthreads();
+  const int pair = threadIdx.x / (2 * T), which = threadIdx.x / T % 2, j = threadIdx.x % T;
+  float* buf = reinterpret_cast<float*>(twl + K::TABN) + threadIdx.x / T * C::SPANP;
   const int nzs = b.nzs[slot];
   const long long nxy = b.nxy;
-  const float2* X = b.ovx[slot] + (long long)y * NX;
-  const float2* Y = X + (long long)b.nzs_stride * nxy;
-  FftTw<NX> twr;
-  __shared__ float2 twstage[NX];
-  load_twiddles(twr, twstage, tid % TPT, tw, tid, NT);
-  double sxr[EPT], sxi[EPT], sx[EPT], sy[EPT];
+  const float2 range = ov_col_range(sup, k, which);
+  const int zskip = sup.bNoKz0 ? sup.zd : -1;  // a plane of zeros, not written
+  const float2* row = b.ovx[slot] + (long long)which * b.nzs_stride * nxy + (long long)y * NX;
+  double pr[HALF], pi[HALF], sx = 0.0, sy = 0.0;
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) sxr[e] = sxi[e] = sx[e] = sy[e] = 0.0;
-  const double n = (double)b.nz;
-  for (int g0 = 0; g0 < nzs; g0 += kOvfG) {
-    const int cnt = nzs - g0 < kOvfG ? nzs - g0 : kOvfG;  // uniform
-    // transform t < kOvfG: X of plane g0 + t; t >= kOvfG: Y of plane g0 + t - kOvfG
-    float2 v[LPT];
+  for (int e = 0; e < HALF; ++e) pr[e] = pi[e] = 0.0;
+  const bool mine = K::ROWS == T || j < K::ROWS;  // the lane ends with outputs
+#pragma unroll 1
+  for (int z0 = 0; z0 < nzs; z0 += pairs) {
+    const int z = z0 + pair;
+    const bool there = pair < pairs && z < nzs && z != zskip;
+    const float2* src = row + (long long)(there ? z : 0) * nxy;
+    float2 in[K::R1 * N1];
 #pragma unroll
-    for (int k = 0; k < LPT; ++k) {
-      const int idx = tid + k * NT;
-      const int t = idx / NX, x = idx % NX;
-      const int pl = t < kOvfG ? t : t - kOvfG;
-      const float2* src = t < kOvfG ? X : Y;
-      v[k] = src[(long long)(g0 + (pl < cnt ? pl : 0)) * nxy + x];
+    for (int c = 0; c < K::R1; ++c) {
+      const int n2 = N2 % T == 0 || j + T * c < N2 ? j + T * c : N2 - 1;
+#pragma unroll
+      for (int n1 = 0; n1 < N1; ++n1) {
+        const int x = N2 * n1 + n2;
+        in[c * N1 + n1] = make_float2(0.f, 0.f);
+        if (there && ov_col_live(sup, range, x)) in[c * N1 + n1] = src[x];
+      }
     }
-    __syncthreads();  // the previous round's reads of lds are done
+    float2 out[N2], v[2 * HALF];
+    rp_transform<NX, 1, true, true, C::WANT>(buf, j, false, twl, in, out);
+    rp_sync<true>();
 #pragma unroll
-    for (int k = 0; k < LPT; ++k) {
-      const int idx = tid + k * NT;
-      lds[(idx / NX) * P + lds_swz<NX>(idx % NX)] = v[k];
+    for (int e = 0; e < 2 * HALF; ++e) v[e] = e < N2 ? out[e] : make_float2(0.f, 0.f);
+#pragma unroll
+    for (int e = 0; e < HALF; ++e) {
+      ov_swap<T>(v[e].x, v[e + HALF].x);
+      ov_swap<T>(v[e].y, v[e + HALF].y);
     }
-    __syncthreads();
-    fft_lds<NX, true>(lds + (tid / TPT) * P, tid % TPT, twr);
+    if (mine) {
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const int x = tid + e * NT;
-      if (x < NX) {
-        const int xs = lds_swz<NX>(x);
-        for (int k = 0; k < cnt; ++k) {
-          const float2 xa = lds[k * P + xs], yb = lds[(kOvfG + k) * P + xs];
-          const double ar = xa.x, ai = xa.y, br = yb.x, bi = yb.y;
-          // float x float products are exact in double: a product plus a
-          // fused multiply-add is the correctly rounded a*b + c*d
-          sxr[e] += __builtin_fma(ar, br, ai * bi);
-          sxi[e] += __builtin_fma(ar, bi, -(ai * br));
-          sx[e] += __builtin_fma(ar, ar, ai * ai);
-          sy[e] += __builtin_fma(br, br, bi * bi);
-        }
+      for (int e = 0; e < HALF; ++e) {
+        const double ar = v[e].x, ai = v[e].y, br = v[e + HALF].x, bi = v[e + HALF].y;
+        // float x float products are exact in double: a product plus a
+        // fused multiply-add is the correctly rounded a*b + c*d
+        pr[e] += __builtin_fma(ar, br, ai * bi);
+        pi[e] += __builtin_fma(ar, bi, -(ai * br));
+        sx += __builtin_fma(ar, ar, ai * ai);
+        sy += __builtin_fma(br, br, bi * bi);
       }
     }
   }
-  double2* Pout = b.P[slot] + (long long)y * NX;
-  double tsx = 0.0, tsy = 0.0;
+  // the pairs' sums, pairwise; entry e of this lane is output x0 + ROWS e
+  const int x0 = j + (which ? K::ROWS * HALF : 0);
+  double2* const sums = reinterpret_cast<double2*>(twl + K::TABN);
+#pragma unroll 1
+  for (int n = pairs; n > 1; n = (n + 1) / 2) {
+    const int half = (n + 1) / 2;
+    __syncthreads();
+    if (pair >= half && pair < n && mine) {
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) {
-    const int x = tid + e * NT;
-    if (x < NX) {
-      const double2 pv = make_double2(sxr[e] * n, sxi[e] * n);
-      Pout[x] = pv;
-      if (b.cc[slot]) b.cc[slot][(long long)y * NX + x] = make_float2((float)pv.x, -(float)pv.y);
-      tsx += sx[e] * n;
-      tsy += sy[e] * n;
+      for (int e = 0; e < HALF; ++e)
+        if (N2 % 2 == 0 || x0 + K::ROWS * e < NX) sums[(pair - half) * NX + x0 + K::ROWS * e] = make_double2(pr[e], pi[e]);
+    }
+    __syncthreads();
+    if (pair + half < n && mine) {
+#pragma unroll
+      for (int e = 0; e < HALF; ++e)
+        if (N2 % 2 == 0 || x0 + K::ROWS * e < NX) {
+          const double2 t = sums[pair * NX + x0 + K::ROWS * e];
+          pr[e] += t.x;
+          pi[e] += t.y;
+        }
     }
   }
-  const double a = block_sum_d<NT>(tsx, red);
-  const double c = block_sum_d<NT>(tsy, red);
-  if (tid == 0) {
-    b.totals[slot][y] = a;
-    b.totals[slot][gridDim.x + y] = c;
+  const double n = (double)b.nz;
+  if (pair == 0 && mine) {
+#pragma unroll
+    for (int e = 0; e < HALF; ++e) {
+      if (N2 % 2 && x0 + K::ROWS * e >= NX) continue;
+      const long long at = (long long)y * NX + x0 + K::ROWS * e;
+      const double2 pv = make_double2(pr[e] * n, pi[e] * n);
+      b.P[slot][at] = pv;
+      if (b.cc[slot]) b.cc[slot][at] = make_float2((float)pv.x, -(float)pv.y);
+    }
+  }
+  const double wx = wave_total(sx), wy = wave_total(sy);
+  if (threadIdx.x % 64 == 0) {
+    red[0][threadIdx.x / 64] = wx;
+    red[1][threadIdx.x / 64] = wy;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double t = 0.0;
+    for (int w = 0; w < (int)blockDim.x / 64; ++w) t += red[threadIdx.x][w];
+    b.totals[slot][threadIdx.x * gridDim.x + y] = t * n;
   }
 }
 
 template <int NY>
 static bool ovf_cols_launch(const OvBatch& ob, int nzs_max, bool run, hipStream_t s) {
   if constexpr (ovf_cols_ok<NY>()) {
+    using C = OvC<NY>;
     const OvParams& p = ob.p[0];
     const size_t lds = p.otf1.ra ? (size_t)2 * p.otf1.nxotf * sizeof(float2) : 0;
     if (lds > 32 * 1024) return false;
+    const float2* tw = twiddles_rp(NY, C::K::N2);
     if (!run) return true;
-    const dim3 g1(2 * ceil_div(p.nx, ovf_cols_w<NY>()), nzs_max, ob.n), b1(ovf_cols_w<NY>() * fft_tpt(NY));
+    const dim3 g1(2 * ceil_div(p.nx, C::W), nzs_max, ob.n), b1(C::NT);
     if (p.otf1.ra)
-      hipLaunchKernelGGL((k_ovf_cols<NY, true>), g1, b1, lds, s, ob, twiddles(NY));
+      hipLaunchKernelGGL((k_ovf_cols<NY, true>), g1, b1, lds, s, ob, tw);
     else
-      hipLaunchKernelGGL((k_ovf_cols<NY, false>), g1, b1, 0, s, ob, twiddles(NY));
+      hipLaunchKernelGGL((k_ovf_cols<NY, false>), g1, b1, 0, s, ob, tw);
     SIMR_LAUNCH_CHECK();
     return true;
   } else {
@@ -583,8 +697,14 @@ static bool ovf_cols_launch(const OvBatch& ob, int nzs_max, bool run, hipStream_
 template <int NX>
 static bool ovf_rows_launch(const ZsumBatch& zb, int ny, bool run, hipStream_t s) {
   if constexpr (ovf_rows_ok<NX>()) {
+    using C = OvR<NX>;
+    const float2* tw = twiddles_rp(NX, C::K::N2);
     if (!run) return true;
-    hipLaunchKernelGGL(k_ovf_rows<NX>, dim3(ny, zb.n), dim3(2 * kOvfG * fft_tpt(NX)), 0, s, zb, twiddles(NX));
+    int nzs = 1;
+    for (int k = 0; k < zb.n; ++k) nzs = std::max(nzs, zb.nzs[k]);
+    // as many pairs as share the planes evenly, at most MAXP
+    const int pairs = ceil_div(nzs, ceil_div(nzs, C::MAXP));
+    hipLaunchKernelGGL(k_ovf_rows<NX>, dim3(ny, zb.n), dim3(C::threads(pairs)), C::lds(pairs), s, zb, pairs, tw);
     SIMR_LAUNCH_CHECK();
     return true;
   } else {
@@ -600,19 +720,25 @@ static int ovf_nzs_max(const OvBatch& ob) {
 
 static bool ovf_cols_dispatch(const OvBatch& ob, bool run, hipStream_t s) {
   switch (ob.p[0].ny) {
-    case 256: return ovf_cols_launch<256>(ob, ovf_nzs_max(ob), run, s);
-    case 512: return ovf_cols_launch<512>(ob, ovf_nzs_max(ob), run, s);
-    case 1024: return ovf_cols_launch<1024>(ob, ovf_nzs_max(ob), run, s);
-    default: return false;
+#define SIMR_CASE(N) \
+  case N:            \
+    return ovf_cols_launch<N>(ob, ovf_nzs_max(ob), run, s);
+    SIMR_XY_SIZES(SIMR_CASE)
+#undef SIMR_CASE
+    default:
+      return false;
   }
 }
 
 static bool ovf_rows_dispatch(const ZsumBatch& zb, int nx, int ny, bool run, hipStream_t s) {
   switch (nx) {
-    case 256: return ovf_rows_launch<256>(zb, ny, run, s);
-    case 512: return ovf_rows_launch<512>(zb, ny, run, s);
-    case 1024: return ovf_rows_launch<1024>(zb, ny, run, s);
-    default: return false;
+#define SIMR_CASE(N) \
+  case N:            \
+    return ovf_rows_launch<N>(zb, ny, run, s);
+    SIMR_XY_SIZES(SIMR_CASE)
+#undef SIMR_CASE
+    default:
+      return false;
   }
 }
 

@@ -230,6 +230,7 @@ Engine::Engine(const simr_params& p, const float* otf, int device) : P(p), L(Lay
   // zoomed assembly lengths), so that no launch path allocates one
   for (int n : {L.nx, L.ny, L.nz, L.xdim, L.ydim, L.zdim})
     if (n > 1) (void)twiddles(n);
+  for (int n : {L.ny, L.nz}) fft_cols_request_table(n);
   {
     AsmParams a{};
     a.nx = L.nx;

@@ -18,9 +18,11 @@ bool fft_size_supported(int n);
 
 // In-place column transforms of length n: element i of column c of plane p at
 // data[p * plane_stride + i * pitch + c] for c < ncols, p < nplanes.
-// tw: the length's twiddle table (nullptr: the cached twiddles(n)).
+// tw: the length's twiddles(n) in caller memory (nullptr: cached tables).
 void fft_cols(int n, float2* data, long long pitch, long long ncols, long long nplanes, long long plane_stride,
               bool inverse, hipStream_t s, const float2* tw = nullptr);
+// Requests the table fft_cols(n, ..., nullptr) takes (as twiddles()).
+void fft_cols_request_table(int n);
 // In-place row transforms: row r (< nrows) at data[r * pitch], n contiguous elements.
 void fft_rows(int n, float2* data, long long pitch, long long nrows, bool inverse, hipStream_t s,
               const float2* tw = nullptr);

@@ -8,6 +8,7 @@
 #include "fft.hpp"
 #include "fft2.hpp"
 #include "fft_api.hpp"
+#include "fft_rp.hpp"
 
 namespace simr {
 
@@ -268,9 +269,76 @@ __global__ __launch_bounds__(W* fft2_tpt(N)) void k_fft2_rows(float2* __restrict
   }
 }
 
+// Columns of lengths whose factors do not pair up for the two-pass core above
+// (N1 | N2), 96 to 640 points: the general two-pass register core, T lanes to a
+// column, W adjacent columns (whole 128-byte lines) to a workgroup.  Bound by
+// HBM; the radix stages below keep the whole tile in LDS and pass through it
+// once a stage, which leaves fewer loads in flight (a quarter to a half of the
+// wavefronts at these lengths).  Forward y transform per launch, before and now:
+// 480x400x21 67.9 and 55.9 us, 384x384x26 64.3 and 61.5 (0.23 GB each way: 90 at
+// the rate of a copy for both launches, now 123), 480x360 9.7 and 7.0.  Longer
+// columns would hold more values a lane than three wavefronts leave room for.
+// A caller's own table (fft_cols' tw) has the radix stages' layout and stays there.
+template <int N>
+constexpr int rpc_want() {
+  return rp_ok(N, 1, kRpWants[1]) ? 1 : 2;
+}
+template <int N>
+constexpr bool rp_cols_ok() {
+  return !use_fft2<N>() && N >= 96 && N <= 640 && rp_ok(N, 1, kRpWants[rpc_want<N>()]);
+}
+template <int N>
+struct RpC {
+  using K = Rp<N, 1, rpc_want<N>()>;
+  static constexpr int W = 16, NT = W * K::T;
+  static constexpr int SPANP = K::SPAN + ((2 - K::SPAN % 32) % 32 + 32) % 32;  // columns two banks apart
+  static constexpr int WAVES = K::R1 * K::N1 > 24 || K::N2 > 24 ? 3 : 4;
+};
+template <int N, bool INV>
+__global__ __launch_bounds__(RpC<N>::NT, RpC<N>::WAVES) void k_rp_cols(float2* __restrict__ data, long long pitch,
+                                                                      long long ncols, long long plane_stride,
+                                                                      const float2* __restrict__ tw) {
+  using C = RpC<N>;
+  using K = typename C::K;
+  constexpr int W = C::W, N1 = K::N1, N2 = K::N2;
+  static_assert(C::NT % 64 == 0 && C::NT <= 1024, "whole wavefronts");
+  __shared__ float buf[W * C::SPANP];
+  unsigned bx, by;
+  xcd_tile(bx, by);
+  const int w = threadIdx.x % W, j = threadIdx.x / W;
+  const long long c = (long long)bx * W + w;
+  float2* col = data + (long long)by * plane_stride + (c < ncols ? c : ncols - 1);
+  float2 in[K::R1 * N1], out[N2];
+#pragma unroll
+  for (int r = 0; r < K::R1; ++r) {
+    const int n2 = N2 % K::T == 0 || j + K::T * r < N2 ? j + K::T * r : N2 - 1;
+#pragma unroll
+    for (int n1 = 0; n1 < N1; ++n1) in[r * N1 + n1] = col[(long long)(N2 * n1 + n2) * pitch];
+  }
+  // (its barriers lie between every load of the tile and every store)
+  rp_transform<N, 1, INV, false, rpc_want<N>()>(buf + w * C::SPANP, j, false, tw, in, out);
+  if (c < ncols && (K::ROWS == K::T || j < K::ROWS)) {
+#pragma unroll
+    for (int k2 = 0; k2 < N2; ++k2) col[(long long)(j + K::ROWS * k2) * pitch] = out[k2];
+  }
+}
+
 template <int N>
 static void launch_cols(float2* data, long long pitch, long long ncols, long long nplanes,
                         long long plane_stride, bool inverse, hipStream_t s, const float2* tw) {
+  if constexpr (rp_cols_ok<N>()) {
+    if (!tw) {
+      using C = RpC<N>;
+      const float2* twr = twiddles_rp(N, C::K::N2);
+      const dim3 grid(ceil_div(ncols, C::W), (unsigned)nplanes);
+      if (inverse)
+        hipLaunchKernelGGL((k_rp_cols<N, true>), grid, dim3(C::NT), 0, s, data, pitch, ncols, plane_stride, twr);
+      else
+        hipLaunchKernelGGL((k_rp_cols<N, false>), grid, dim3(C::NT), 0, s, data, pitch, ncols, plane_stride, twr);
+      SIMR_LAUNCH_CHECK();
+      return;
+    }
+  }
   if (!tw) tw = twiddles(N);
   if constexpr (use_fft2<N>()) {
     constexpr int W = tile_w2<N>();
@@ -349,6 +417,26 @@ void fft_cols(int n, float2* data, long long pitch, long long ncols, long long n
 #undef SIMR_CASE
     default:
       throw ArgError("FFT length " + std::to_string(n) + " is not supported (must be 2^a 3^b 5^c, <= 4096)");
+  }
+}
+
+template <int N>
+static void request_cols_table() {
+  if constexpr (rp_cols_ok<N>())
+    (void)twiddles_rp(N, RpC<N>::K::N2);
+  else
+    (void)twiddles(N);
+}
+void fft_cols_request_table(int n) {
+  switch (n) {
+#define SIMR_CASE(N)         \
+  case N:                    \
+    request_cols_table<N>(); \
+    return;
+    SIMR_FFT_SIZES(SIMR_CASE)
+#undef SIMR_CASE
+    default:
+      return;
   }
 }
 

@@ -231,6 +231,7 @@ Engine::Engine(const simr_params& p, const float* otf, int device) : P(p), L(Lay
   for (int n : {L.nx, L.ny, L.nz, L.xdim, L.ydim, L.zdim})
     if (n > 1) (void)twiddles(n);
   for (int n : {L.ny, L.nz}) fft_cols_request_table(n);
+  overlaps_request_tables(L.nx, L.ny);
   {
     AsmParams a{};
     a.nx = L.nx;
@@ -814,9 +815,9 @@ ModampSlots Engine::modamp_slots() const {
 
 // Queues the modamp reductions of n <= kMaxCand candidates (direction,
 // vector) at entries [at, at + n) of the zero-copy region: the candidates
-// travel in the kernel arguments, and the partials are summed per candidate in
-// block order on the device as the host does (cpuReduce,
-// gpuFunctionsImpl_hh.cu:162-180), straight into the region.  The sums are
+// travel in the kernel arguments, and the partials are summed per candidate on
+// the device (FP32 fit: in block order as cpuReduce, gpuFunctionsImpl_hh.cu:162-180;
+// FP64: in wave_sum's order), straight into the region.  The sums are
 // read (eval_read) after the next wait_fit().
 void Engine::eval_enqueue(const Cand* c, int n, int at) {
   SIMR_REQUIRE(n >= 1 && n <= kMaxCand && at >= 0 && at + n <= kZcCand, "modamp batch out of range");

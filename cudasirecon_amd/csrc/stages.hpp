@@ -123,8 +123,11 @@ void launch_overlaps_z_reduce(const ZsumBatch& b, bool fp32, bool per_elem, hipS
 // inverse x transform with the z sums (by rows, ..._rows); P and the totals
 // as launch_overlaps_z_reduce(fp32 = false, per_elem = false) leaves them.
 // overlaps_fused_ok: whether the geometry is covered.
-OvSupport ov_support(const OvParams& p);
 bool overlaps_fused_ok(const OvBatch& ob, const ZsumBatch& zb);
+// The twiddle tables of both passes (as twiddles()).
+void overlaps_request_tables(int nx, int ny);
+// What the row pass needs of a slot to know the columns the first leaves unwritten.
+OvSupport ov_support(const OvParams& p);
 void launch_overlaps_fused_cols(const OvBatch& ob, hipStream_t s);
 void launch_overlaps_fused_rows(const ZsumBatch& zb, int nx, int ny, hipStream_t s);
 // Inverse z DFT of the stored kz planes of both overlaps into real-space

@@ -756,6 +756,16 @@ bool overlaps_fused_ok(const OvBatch& ob, const ZsumBatch& zb) {
   return ovf_cols_dispatch(ob, false, nullptr) && ovf_rows_dispatch(zb, p0.nx, p0.ny, false, nullptr);
 }
 
+void overlaps_request_tables(int nx, int ny) {
+  OvBatch ob{};
+  ZsumBatch zb{};
+  ob.n = zb.n = 1;
+  ob.p[0].nx = nx;
+  ob.p[0].ny = ny;
+  (void)ovf_cols_dispatch(ob, false, nullptr);
+  (void)ovf_rows_dispatch(zb, nx, ny, false, nullptr);
+}
+
 void launch_overlaps_fused_cols(const OvBatch& ob, hipStream_t s) {
   if (!ovf_cols_dispatch(ob, true, s)) throw ArgError("two-pass overlaps: unsupported geometry");
 }

@@ -1268,7 +1268,7 @@ bool Engine::fit_on_device() {
   reqs.clear();
   for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, 0, fo2, 0.f, 0.f, &fitst_->d[d].kov, (float)fo2});
   make_overlaps(reqs);
-  const ModampSlots ms = modamp_slots();
+  const ModampSlots ms = modamp_slots();  // of the overlaps just queued
   CandSet cs{};
   cs.kc = fitst_->kc;
   cs.nreq = fitst_->nreq;
@@ -1611,11 +1611,11 @@ void Engine::build_graph() {
   SIMR_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
   try {
     const int nparts = fit_fp32_ ? modamp_partials_fp32(L.nx, L.ny) : modamp_partials_fp64(L.nx, L.ny);
-    const ModampSlots m = modamp_slots();
     for (int o = 1; o < L.norders; ++o) {
       std::vector<OvReq> reqs;
       for (int d = 0; d < L.ndirs; ++d) reqs.push_back({d, 0, o, k0_[d].x, k0_[d].y});
       make_overlaps(reqs);
+      const ModampSlots m = modamp_slots();  // (the partials' count is these overlaps')
       CandSet cs{};
       cs.kc = kc_dev_ + (size_t)o * L.ndirs;
       cs.ks = slot_ids_;

@@ -261,7 +261,7 @@ void launch_fit_begin(FitState* fs, const FitArgs& a, const float2* cc, const fl
 void launch_fit_walk(FitState* fs, const FitArgs& a, const ModampSlots& m, const double2* part64, int nparts,
                      float2* amps, float* corr, const FitPub& pub, hipStream_t s);
 // findrealspacemodamp's result (gpuFunctionsImpl.cu:1128-1147) on the device,
-// for each of ncand candidates (one per slot): the partials summed as
+// for candidates c = 0 .. ncand - 1, of slot kslot[c] = c: the partials summed as
 // launch_modamp_evals does, then modamp = XStarY / sumX and corr =
 // |XStarY| / sqrt(sumX sumY), written to amp[kslot[c] * stride + order] and
 // corr[same].  fp64: part64 [ncand][nparts] and the slot's z-sum totals;

@@ -1084,6 +1084,13 @@ static void check_cands(const CandSet& c, int ncand) {
   if (c.nreq == nullptr && (c.kc == nullptr) != (c.ks == nullptr)) throw ArgError("modamp: candidates and slots from the same source");
 }
 
+// The z-sum totals of a slot that is read must have been queued: zb is 0 until
+// its overlaps are.
+static void check_totals(const ModampSlots& m, int slot) {
+  if (slot < 0 || slot >= kMaxDirs || m.zb[slot] < 1 || m.zb[slot] > kZsumMaxBlocks)
+    throw ArgError("modamp: a direction without overlaps");
+}
+
 void launch_modamp_fp64(const ModampSlots& m, const CandSet& c, int ncand, int nx, int ny, float dxy,
                         double2* partials, hipStream_t s) {
   check_cands(c, ncand);
@@ -1165,6 +1172,7 @@ void launch_modamp_finish(bool fp32, const ModampSlots& m, const int* kslot, int
                        order);
     if (pub.out != nullptr) hipLaunchKernelGGL(k_fit_publish, dim3(1), dim3(64), 0, s, fit, pub, amp, corr);
   } else {
+    for (int k = 0; k < ncand; ++k) check_totals(m, k);  // kslot holds slots 0 .. ncand - 1
     hipLaunchKernelGGL(k_modamp_finish_fp64, dim3(1), dim3(64 * ncand), 0, s, m, kslot, ncand, part64, nparts, amp,
                        corr, stride, order, fit, pub);
   }
@@ -1208,6 +1216,8 @@ __global__ __launch_bounds__(256) void k_modamp_evals(int fp32, ModampSlots m, C
 void launch_modamp_evals(bool fp32, const ModampSlots& m, const CandSet& c, int ncand, const double2* part64,
                          const float4* part32, int nparts, double* out, bool host_out, hipStream_t s) {
   check_cands(c, ncand);
+  if (!fp32)
+    for (int k = 0; k < ncand && c.kc == nullptr; ++k) check_totals(m, c.slot[k]);
   hipLaunchKernelGGL(k_modamp_evals, dim3(ncand), dim3(256), 0, s, fp32 ? 1 : 0, m, c, part64, part32, nparts, out,
                      host_out ? 1 : 0);
   SIMR_LAUNCH_CHECK();

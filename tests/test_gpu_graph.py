@@ -104,3 +104,56 @@ def test_graph_recaptured_after_parameter_change():
     out = run_pair(p, otf, frames, update_at=3)
     assert_same(out, p.ndirs, 3)
     assert not np.array_equal(out["g"][2][0], out["g"][3][0])
+
+
+def time_point(r, raw, t):
+    r.set_raw(raw)
+    r.load_and_rescale(t)
+    r.set_time(t)
+    r.process_volume()
+    return r.result(), [r.fit(d) for d in range(r.p.ndirs)]
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 8, 5), (128, 96, 1, 3), (64, 40, 8, 5)])
+@pytest.mark.parametrize("fit64", [True, False])
+def test_first_graphed_time_point_of_a_context_with_another_ones_state(shape, fit64):
+    """A context that takes over another context's time-0 state captures its graph before it has
+    built any overlaps: its time points equal the sequential eager context's bit for bit."""
+    log("case: time-0 state of %s into a fresh graphed context, fit64=%d" % (shape, fit64))
+    p, otf, frames = frames_of(54, 3, shape=shape)
+    p.ntimes, p.fit_fp64 = len(frames), int(fit64)
+    qg, qe = p.copy(), p.copy()
+    qg.use_graphs, qe.use_graphs = 1, 0
+    lib = engine.lib()
+    with engine.Reconstructor(qe, otf) as e, engine.Reconstructor(qg, otf) as g:
+        time_point(e, frames[0], 0)
+        n = lib.simr_time0_state_size(e.h)
+        state = engine.C.create_string_buffer(n)
+        engine._check(lib.simr_get_time0_state(e.h, state, n))
+        engine._check(lib.simr_set_time0_state(g.h, state, n))
+        out = {"g": [], "e": []}
+        for t in (1, 2):
+            out["g"].append(time_point(g, frames[t], t))
+            out["e"].append(time_point(e, frames[t], t))
+        assert np.isfinite(out["g"][0][0]).all()
+        assert_same(out, p.ndirs, shape[3] // 2 + 1)
+
+
+@pytest.mark.parametrize("first64", [False, True])
+def test_graph_after_a_change_of_the_fit_precision(first64):
+    """Time 0 in one precision, the later time points in the other: the z sums that the captured
+    modamps read come in other partials than time 0's did."""
+    log("case: 3-frame 64x64x8 series, fit_fp64 %d at t=0, %d after" % (first64, not first64))
+    p, otf, frames = frames_of(55, 3, shape=(64, 64, 8, 5))
+    p.ntimes, p.fit_fp64 = len(frames), int(first64)
+    qg, qe = p.copy(), p.copy()
+    qg.use_graphs, qe.use_graphs = 1, 0
+    out = {"g": [], "e": []}
+    with engine.Reconstructor(qg, otf) as g, engine.Reconstructor(qe, otf) as e:
+        for t, raw in enumerate(frames):
+            for key, r, q in (("g", g, qg), ("e", e, qe)):
+                if t == 1:
+                    q.fit_fp64 = int(not first64)
+                    engine._check(engine.lib().simr_update_params(r.h, engine.C.byref(q)))
+                out[key].append(time_point(r, raw, t))
+    assert_same(out, p.ndirs, 3)

@@ -365,10 +365,16 @@ __device__ __forceinline__ float2 ov_shift(const OvSupport& q) {
 // nonzero element: those whose frequency lies in the x extent of the lens
 // |q| <= rc, |q - s| <= rc (s = k, or -k for overlap1).  Its rightmost point is
 // one disc's, if that lies in the other disc, else the discs' right
-// intersection; likewise on the left.  The range carries a margin far beyond
-// the rounding of the per-element tests; hi < lo: no column.  (Plane kz = 0
-// with bNoKz0 is left to the callers.)
-__device__ __forceinline__ float2 ov_col_range(const OvSupport& p, float2 k, int which) {
+// intersection; likewise on the left.  The range carries a margin of
+// margin * r, far beyond the rounding of the per-element tests; hi < lo: no
+// column.  The column pass writes the tiles that meet the range with
+// kOvWritten, and the row pass reads the columns in the range with kOvRead:
+// the difference is far beyond the rounding of the range in either kernel, so
+// no column is read that was not written.  (Plane kz = 0 with bNoKz0 is left
+// to the callers.)
+constexpr float kOvWritten = 1e-3f, kOvRead = 0.5e-3f;
+__device__ __forceinline__ float2 ov_col_range(const OvSupport& p, float2 k, int which, float margin) {
+#pragma clang fp contract(off)
   const float sx = which == 0 ? k.x : -k.x, sy = which == 0 ? k.y : -k.y;
   const float r2 = p.rc2 * 1.0002f, r = __builtin_amdgcn_sqrtf(r2);
   const float d2 = sx * sx + sy * sy;
@@ -379,10 +385,11 @@ __device__ __forceinline__ float2 ov_col_range(const OvSupport& p, float2 k, int
   // the right end of the disc further left, if inside the other; else the intersection
   const float e2 = (r - fabsf(sx)) * (r - fabsf(sx)) + sy * sy;  // its squared distance from the other's centre
   const float half = e2 <= r2 ? r - 0.5f * fabsf(sx) : chord;    // the lens is symmetric about s / 2
-  const float m = 1e-3f * r;
+  const float m = margin * r;
   return make_float2(0.5f * sx - half - m, 0.5f * sx + half + m);
 }
 __device__ __forceinline__ bool ov_col_live(const OvSupport& p, float2 range, int j) {
+#pragma clang fp contract(off)
   const float x = (float)(j > p.nx / 2 ? j - p.nx : j) * p.dkx;
   return x >= range.x && x <= range.y;
 }
@@ -449,7 +456,7 @@ __global__ __launch_bounds__(OvC<NY>::NT, OvC<NY>::WAVES) void k_ovf_cols(OvBatc
   const OvSupport sup{p.kx, p.ky, p.k0d, p.kmul, p.rc2, p.dkx, p.dky, p.nx, p.ny, p.zd, p.bNoKz0};
   const float2 k = ov_shift(sup);
   {
-    const float2 range = ov_col_range(sup, k, which);
+    const float2 range = ov_col_range(sup, k, which, kOvWritten);
     bool live = false;
     for (int w = 0; w < W; ++w) live = live || (c0 + w < p.nx && ov_col_live(sup, range, c0 + w));
     if (!live) return;  // uniform over the workgroup
@@ -580,7 +587,7 @@ __global__ __launch_bounds__(OvR<NX>::threads(OvR<NX>::MAXP), OvR<NX>::WAVES) vo
   float* buf = reinterpret_cast<float*>(twl + K::TABN) + threadIdx.x / T * C::SPANP;
   const int nzs = b.nzs[slot];
   const long long nxy = b.nxy;
-  const float2 range = ov_col_range(sup, k, which);
+  const float2 range = ov_col_range(sup, k, which, kOvRead);
   const int zskip = sup.bNoKz0 ? sup.zd : -1;  // a plane of zeros, not written
   const float2* row = b.ovx[slot] + (long long)which * b.nzs_stride * nxy + (long long)y * NX;
   double pr[HALF], pi[HALF], sx = 0.0, sy = 0.0;

@@ -44,3 +44,32 @@ def test_fit_overlaps_in_two_passes(nx, ny, nz, kw):
             print("  direction %d: modamp off by %.1e" % (d, abs(got - want) / abs(want)), flush=True)
             assert abs(got - want) < 2e-6 * abs(want)
             assert abs(f.corr[1] - cc) < 2e-6 * cc
+
+
+@pytest.mark.parametrize("nx,ny,nz,phases,kw", [(64, 64, 24, 5, {}), (200, 100, 12, 5, {}), (512, 96, 8, 5, {}),
+                                                (128, 80, 1, 3, {}), (480, 48, 9, 5, dict(bNoKz0=1))])
+def test_nothing_unwritten_is_read(nx, ny, nz, phases, kw):
+    """The column pass leaves columns without an element unwritten and the row pass leaves them
+    unread: staging memory full of NaN (a stack of NaN, whose overlap volumes go there) changes
+    nothing in the next reconstruction."""
+    print("case %dx%dx%d, %d phases, %s, staging full of NaN" % (nx, ny, nz, phases, kw), flush=True)
+    p, otf, raw, _ = synthetic(nx, ny, nz, nphases=phases, seed=nx + ny, gpu=True, zoomfact=2.0, **kw)
+
+    def once(r):
+        r.set_raw(raw)
+        r.load_and_rescale(0)
+        r.set_time(0)
+        r.process_volume()
+        return r.result(), [r.fit(d) for d in range(p.ndirs)]
+
+    with engine.Reconstructor(p, otf) as r, engine.Reconstructor(p, otf) as fresh:
+        r.set_raw(np.full(raw.shape, np.nan, np.float32))
+        r.load_and_rescale(0)
+        for d in range(p.ndirs):
+            ov = r.overlap_volumes(d, 0, 1, 1.0, 0.5)
+        assert np.isnan(ov[0]).all() and np.isnan(ov[1]).all()
+        got, fits = once(r)
+        want, wfits = once(fresh)
+        assert np.isfinite(want).all() and np.array_equal(got, want)
+        for f, w in zip(fits, wfits):
+            assert (f.k0x, f.k0y, list(f.amp_re), list(f.corr)) == (w.k0x, w.k0y, list(w.amp_re), list(w.corr))

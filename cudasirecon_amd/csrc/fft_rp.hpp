@@ -113,6 +113,27 @@ struct Rp {
   static constexpr int OSTEP = SPLIT ? 2 * N1 : ROWS;
 };
 
+// Wavefronts per SIMD that a lane's values (a pass's inputs or outputs) leave
+// room for beside the sums and addresses of the assembly passes.
+constexpr int rp_waves(int values) { return values <= 32 ? 3 : values <= 40 ? 2 : 1; }
+template <int LEN, int HALVES>
+constexpr int rp_values() {
+  using K = Rp<LEN, HALVES>;
+  return K::R1 * K::HL * K::N1 > K::N2 ? K::R1 * K::HL * K::N1 : K::N2;
+}
+// Whether a transform of N points with fewer than N/2 of them occupied (a zoom
+// above two) is better done as the halves of an N/2-point one, with the empty
+// frequencies as zeros in its input, than whole: where the halves' plan leaves
+// room for more wavefronts, and for long ones where a lane forms both halves.
+// Assembly x pass, whole and as halves, 6 planes: 1536 points (384 columns) 490
+// and 297 us, 1920 (480) 807 and 414, 2048 (512) 910 and 392, 2304 (576) 1086 and
+// 985, 2880 (720) 1677 and 1263; without more room 3072 points (768) take 1746
+// and 2115, 4096 (1024) 2824 and 3662.
+template <int N>
+constexpr bool rp_halves_pay() {
+  return rp_waves(rp_values<N / 2, 2>()) > rp_waves(rp_values<N, 1>()) || (N > 1024 && Rp<N / 2, 2>::HL == 2);
+}
+
 // o[n1] = v[n1] exp(+-i pi n1 / N1), negated where the frequency of element
 // N2 n1 + n2 of the M-point input is negative (index above M/2)
 template <int LEN, bool INV, int N1I = 0>

@@ -317,7 +317,7 @@ struct AsmY {
   static constexpr int LDS = lds_of(W);
 };
 
-template <int N, int HALVES>
+template <int N, int HALVES, bool PAD>
 __global__ __launch_bounds__((AsmY<N, HALVES>::NT), (AsmY<N, HALVES>::WAVES)) void k_asm_y(AsmParams p, const float2* __restrict__ tw) {
   using C = AsmY<N, HALVES>;
   using K = typename C::K;
@@ -360,11 +360,11 @@ __global__ __launch_bounds__((AsmY<N, HALVES>::NT), (AsmY<N, HALVES>::WAVES)) vo
       // frequency of element n, and its source row (centred: row y + hy)
       int y;
       bool live = true;
-      if (HALVES == 2) {
+      if (HALVES == 2 && !PAD) {
         y = n > LEN / 2 ? n - LEN : n;
       } else {
-        const bool lo = n <= p.ny - p.ny / 2, hi = n >= N - hy;
-        y = lo ? n : n - N;
+        const bool lo = n <= p.ny - p.ny / 2, hi = n >= LEN - hy;
+        y = lo ? n : n - LEN;
         live = lo || hi;
       }
       live = live && !asm_dead(p, xc - (p.nx / 2 - 1), y, p.rc2_zero * 0.9999f);
@@ -482,12 +482,12 @@ void launch_asm_z(const AsmParams& p, hipStream_t s) {
 }
 
 // The y pass at zoomed height N; run = false only requests its twiddle table.
-template <int N, int HALVES>
+template <int N, int HALVES, bool PAD>
 static void launch_asm_y_n(const AsmParams& p, bool run, hipStream_t s) {
   using C = AsmY<N, HALVES>;
   const float2* tw = twiddles_rp(N, C::K::N2);
   if (!run) return;
-  hipLaunchKernelGGL((k_asm_y<N, HALVES>), dim3(ceil_div(p.nx, C::W), p.zdim, p.nasm), dim3(C::NT), 0, s, p, tw);
+  hipLaunchKernelGGL((k_asm_y<N, HALVES, PAD>), dim3(ceil_div(p.nx, C::W), p.zdim, p.nasm), dim3(C::NT), 0, s, p, tw);
   SIMR_LAUNCH_CHECK();
 }
 
@@ -496,9 +496,11 @@ static void asm_y_dispatch(const AsmParams& p, bool run, hipStream_t s) {
 #define SIMR_CASE(N)                            \
   case N:                                       \
     if (2 * p.ny == N)                          \
-      launch_asm_y_n<N, 2>(p, run, s);          \
+      launch_asm_y_n<N, 2, false>(p, run, s);   \
+    else if (2 * p.ny < N && rp_halves_pay<N>()) \
+      launch_asm_y_n<N, 2, rp_halves_pay<N>()>(p, run, s); \
     else                                        \
-      launch_asm_y_n<N, 1>(p, run, s);          \
+      launch_asm_y_n<N, 1, false>(p, run, s);   \
     return;
     SIMR_ZOOM_SIZES(SIMR_CASE)
 #undef SIMR_CASE

@@ -49,15 +49,16 @@ __device__ __forceinline__ float2 asm_phasor(const AsmParams& p, int a, int X, i
   return make_float2(2.f * cs, 2.f * sn);
 }
 
-// The phasors of bands 1 .. nasm-1 at every output column, [band - 1][Y][pos]:
-// pos is the column, or with split halves the even columns and then the odd
-// ones (the order in which the x pass's lanes read them).
-__global__ __launch_bounds__(256) void k_asm_phasors(AsmParams p, int split, float2* __restrict__ lut) {
+// The phasors of bands 1 .. nasm-1 at every column of the output rows y0 + Y,
+// [band - 1][Y][pos]: pos is the column, or with split halves the even columns
+// and then the odd ones (the order in which the x pass's lanes read them).
+__global__ __launch_bounds__(256) void k_asm_phasors(AsmParams p, int split, int y0, float2* __restrict__ lut) {
   const int pos = blockIdx.x * 256 + threadIdx.x;
   if (pos >= p.xdim) return;
   const int half = p.xdim / 2;
   const int X = !split ? pos : pos < half ? 2 * pos : 2 * (pos - half) + 1;
-  lut[((long long)blockIdx.z * p.ydim + blockIdx.y) * p.xdim + pos] = asm_phasor(p, blockIdx.z + 1, X, blockIdx.y);
+  lut[((long long)blockIdx.z * gridDim.y + blockIdx.y) * p.xdim + pos] =
+      asm_phasor(p, blockIdx.z + 1, X, y0 + (int)blockIdx.y);
 }
 
 template <int N, int HALVES>
@@ -66,22 +67,31 @@ struct AsmX {
   using K = Rp<LEN, HALVES>;
   // floats of one slot's LDS: neighbouring slots of a wavefront offset by T banks
   static constexpr int SPANP = K::SPAN + ((K::T - K::SPAN % 64) % 64 + 64) % 64;
-  // twiddles, exchange buffers and, without the phasor table, every lane's phasors of one band
+  // Phasors of one band that a lane forms at a time without the table, behind
+  // the band's transform.  All of them at once, ahead of it, hold 8 bytes of LDS
+  // a value, so that one workgroup fits a CU: one plane of 2560 columns (zoom 2)
+  // 228 -> 141 us, 3072 (zoom 3) 382 -> 201.  The transform's outputs live
+  // meanwhile, so two wavefronts per SIMD are asked for (at three 50 to 74
+  // registers spill).
+  static constexpr int PB = K::N2 < 16 ? K::N2 : 16;
+  // twiddles, exchange buffers and, without the phasor table, every lane's PB phasors
   static constexpr int lds_bytes(int threads, bool lut) {
-    return K::TABN * 8 + threads / K::T * SPANP * 4 + (lut ? 0 : threads * K::N2 * 8);
+    return K::TABN * 8 + threads / K::T * SPANP * 4 + (lut ? 0 : threads * PB * 8);
   }
   static constexpr int MAXT = lds_bytes(256, false) <= 160 * 1024 ? 256 : 128;  // threads per workgroup, at most
   static_assert(lds_bytes(MAXT, false) <= 160 * 1024, "rows, phasors and twiddles fit the LDS");
   static constexpr int MINT = K::SPLIT ? 128 : 64;  // a pair of wavefronts (even, odd half) or one
   // wavefronts per SIMD asked of the register allocator (168 VGPRs each at
   // three, 256 at two)
-  static constexpr int VALUES = K::R1 * K::HL * K::N1 > K::N2 ? K::R1 * K::HL * K::N1 : K::N2;
-  static constexpr int WAVES = VALUES <= 32 ? 3 : VALUES <= 40 ? 2 : 1;
+  static constexpr int waves(bool lut) {
+    const int w = rp_waves(rp_values<LEN, HALVES>());
+    return lut || w < 3 ? w : 2;
+  }
   // rows a workgroup of `threads` takes
   static constexpr int rows(int threads) { return threads / K::T / (K::SPLIT ? 2 : 1); }
 };
 
-template <int N, int HALVES>
+template <int N, int HALVES, bool PAD>
 __device__ __forceinline__ void asm_x_fetch(const AsmParams& p, const float2* src, int j,
                                             float2 (&in)[Rp<N / HALVES, HALVES>::R1 * Rp<N / HALVES, HALVES>::N1]) {
   using K = Rp<N / HALVES, HALVES>;
@@ -94,7 +104,7 @@ __device__ __forceinline__ void asm_x_fetch(const AsmParams& p, const float2* sr
     for (int n1 = 0; n1 < N1; ++n1) {
       const int B = N2 * n1;
       float2& d = in[c * N1 + n1];
-      if constexpr (HALVES == 2) {  // source column of frequency n (n <= LEN/2) or n - LEN
+      if constexpr (HALVES == 2 && !PAD) {  // source column of frequency n (n <= LEN/2) or n - LEN
         if (B > LEN / 2)
           d = src[B - LEN / 2 - 1 + n2];
         else if (B + N2 - 1 <= LEN / 2)
@@ -103,17 +113,18 @@ __device__ __forceinline__ void asm_x_fetch(const AsmParams& p, const float2* sr
           d = src[B + n2 + (B + n2 > LEN / 2 ? -LEN / 2 - 1 : LEN / 2 - 1)];
       } else {
         const int n = B + n2;
-        const bool lo = n <= p.nx - half, hi = n >= N - (half - 1);
-        const float2 t = src[lo ? n + half - 1 : hi ? n - N + half - 1 : 0];
+        const bool lo = n <= p.nx - half, hi = n >= LEN - (half - 1);
+        const float2 t = src[lo ? n + half - 1 : hi ? n - LEN + half - 1 : 0];
         d = lo || hi ? t : make_float2(0.f, 0.f);
       }
     }
   }
 }
 
-template <int N, int HALVES, bool LUT>
-__global__ __launch_bounds__((AsmX<N, HALVES>::MAXT), (AsmX<N, HALVES>::WAVES)) void k_asm_x(AsmParams p, const float2* __restrict__ tw,
-                                                                  const float2* __restrict__ lut) {
+// Output rows y0 .. y0 + ny - 1 of every plane.
+template <int N, int HALVES, bool PAD, bool LUT>
+__global__ __launch_bounds__((AsmX<N, HALVES>::MAXT), (AsmX<N, HALVES>::waves(LUT))) void k_asm_x(
+    AsmParams p, int y0, int ny, const float2* __restrict__ tw, const float2* __restrict__ lut) {
 #pragma clang fp contract(off)
   using C = AsmX<N, HALVES>;
   using K = typename C::K;
@@ -129,32 +140,28 @@ __global__ __launch_bounds__((AsmX<N, HALVES>::MAXT), (AsmX<N, HALVES>::WAVES)) 
   const int rslot = K::SPLIT ? (wave >> 1) * (64 / T) + slot % (64 / T) : slot;
   const unsigned q = gridDim.x / 8u, r8 = gridDim.x % 8u, xcd = blockIdx.x % 8u;  // XCD-contiguous rows
   const long long blk = (long long)xcd * q + (xcd < r8 ? xcd : r8) + blockIdx.x / 8u;
-  const long long nrows = (long long)p.ydim * p.zdim;
+  const long long nrows = (long long)ny * p.zdim;
   const long long row = blk * (blockDim.x / T / (K::SPLIT ? 2 : 1)) + rslot;
   const long long rc = row < nrows ? row : nrows - 1;
-  const int Y = (int)(rc / p.zdim), z = (int)(rc - (long long)Y * p.zdim);
+  const int yl = (int)(rc / p.zdim), z = (int)(rc - (long long)yl * p.zdim);
+  const int Y = y0 + yl;
   const float2* src = p.stageY + ((long long)z * p.ydim + Y) * p.nx;
   const long long band = (long long)p.zdim * p.ydim * p.nx;
   const int jr = K::ROWS == T || j < K::ROWS ? j : K::ROWS - 1;
   const int X0 = K::out0(jr, odd ? 1 : 0);
   // the lane's phasors: entry pos0 + PSTEP k2 of each band's row
   constexpr int PSTEP = K::SPLIT ? N1 : K::ROWS;
-  const float2* ph = LUT ? lut + (long long)Y * N + (K::SPLIT && odd ? N / 2 : 0) + jr : nullptr;
+  const float2* ph = LUT ? lut + (long long)yl * N + (K::SPLIT && odd ? N / 2 : 0) + jr : nullptr;
   float2* phl = reinterpret_cast<float2*>(reinterpret_cast<float*>(twl + K::TABN) + blockDim.x / T * C::SPANP);
   float acc[N2];
 #pragma unroll 1
   for (int a = 0; a < p.nasm; ++a, src += band) {
-    if (!LUT && a > 0) {
-#pragma unroll 1
-      for (int k2 = 0; k2 < N2; ++k2)
-        phl[k2 * blockDim.x + threadIdx.x] = asm_phasor(p, a, X0 + K::OSTEP * k2, Y);
-    }
     float2 in[K::R1 * N1], v[N2];
     int jo = j;
     // keeps the general zoom's per-element offsets from being hoisted out of
     // the band loop into registers
-    if (HALVES == 1) asm volatile("" : "+v"(jo));
-    asm_x_fetch<N, HALVES>(p, src, jo, in);
+    if (HALVES == 1 || PAD) asm volatile("" : "+v"(jo));
+    asm_x_fetch<N, HALVES, PAD>(p, src, jo, in);
     rp_transform<C::LEN, HALVES, true, true>(buf, j, odd, twl, in, v);
     rp_sync<true>();
     // write_outbuffer_kernel1/2, gpuFunctionsImpl.cu:1956-1991: band 0 adds
@@ -167,13 +174,28 @@ __global__ __launch_bounds__((AsmX<N, HALVES>::MAXT), (AsmX<N, HALVES>::WAVES)) 
     if (a == 0) {
 #pragma unroll
       for (int k2 = 0; k2 < N2; ++k2) acc[k2] = 0.f + v[k2].x;
-    } else {
-      const float2* pa = LUT ? ph + (long long)(a - 1) * p.ydim * N : nullptr;
+    } else if constexpr (LUT) {
+      const float2* pa = ph + (long long)(a - 1) * ny * N;
 #pragma unroll
       for (int k2 = 0; k2 < N2; ++k2) {
-        const float2 f = LUT ? pa[PSTEP * k2] : phl[k2 * blockDim.x + threadIdx.x];
+        const float2 f = pa[PSTEP * k2];
         acc[k2] += __builtin_fmaf(v[k2].x, f.x, -(v[k2].y * f.y));
         if (k2 % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // bounds the phasors in flight
+      }
+    } else {
+      constexpr int PB = C::PB;
+#pragma unroll
+      for (int k0 = 0; k0 < N2; k0 += PB) {
+        const int n = N2 - k0 < PB ? N2 - k0 : PB;
+#pragma unroll 1
+        for (int i = 0; i < n; ++i)
+          phl[i * blockDim.x + threadIdx.x] = asm_phasor(p, a, X0 + K::OSTEP * (k0 + i), Y);
+#pragma unroll
+        for (int i = 0; i < PB; ++i) {
+          if (k0 + i >= N2) break;
+          const float2 f = phl[i * blockDim.x + threadIdx.x];
+          acc[k0 + i] += __builtin_fmaf(v[k0 + i].x, f.x, -(v[k0 + i].y * f.y));
+        }
       }
     }
   }
@@ -202,7 +224,7 @@ struct AsmXW {
   static size_t lds_bytes(int nasm) { return (size_t)K::TABN * 8 + (size_t)waves(nasm) * REGION * 4; }
 };
 
-template <int N, int HALVES>
+template <int N, int HALVES, bool PAD>
 __global__ __launch_bounds__(1024) void k_asm_x_wide(AsmParams p, const float2* __restrict__ tw) {
 #pragma clang fp contract(off)
   using C = AsmXW<N, HALVES>;
@@ -223,7 +245,7 @@ __global__ __launch_bounds__(1024) void k_asm_x_wide(AsmParams p, const float2* 
     const int Y = (int)(row / p.zdim), z = (int)(row - (long long)Y * p.zdim);
     const float2* src = p.stageY + (((long long)a * p.zdim + z) * p.ydim + Y) * p.nx;
     float2 in[K::R1 * K::N1], v[N2];
-    asm_x_fetch<N, HALVES>(p, src, j, in);
+    asm_x_fetch<N, HALVES, PAD>(p, src, j, in);
     rp_transform<C::LEN, HALVES, true, true>(reg + slot * AsmX<N, HALVES>::SPANP, j, h != 0, twl, in, v);
     rp_sync<true>();
     // the lane's outputs, read back by the same lane
@@ -255,9 +277,15 @@ __global__ __launch_bounds__(1024) void k_asm_x_wide(AsmParams p, const float2* 
 }
 
 // The x pass at zoomed width N.  The phasor table pays where several planes
-// read each of its rows and the idle z-pass staging holds it; with few
-// planes the phasors are formed in the kernel.
-template <int N, int HALVES>
+// read each of its rows (1, 2 and 3 planes: slower).  It lies in the idle z-pass
+// staging; where that holds some of the output rows only (zoom^2 above the number
+// of planes, about), the pass goes over the rows in parts, if a part fills the
+// device twice over (two of the smallest workgroups per SIMD).  Elsewhere the
+// phasors are formed in the kernel.  1536 columns, zoom 3, 6 planes: 301 us
+// without the table, 238 in parts; 2048, zoom 4: 728 and 392; 120 columns at zoom
+// 8, 9 planes: 187, and 329 in parts of a quarter of that bound.
+constexpr long long kAsmPartGroups = 2048;
+template <int N, int HALVES, bool PAD>
 static void launch_asm_x_n(const AsmParams& p, bool run, hipStream_t s) {
   using C = AsmX<N, HALVES>;
   const float2* tw = twiddles_rp(N, C::K::N2);
@@ -270,27 +298,38 @@ static void launch_asm_x_n(const AsmParams& p, bool run, hipStream_t s) {
     // and share the phasor table.)
     if (ceil_div(nrows, W::rows()) * (C::K::SPLIT ? 2 : 1) <= 1024 && p.nasm > 1 && W::waves(p.nasm) <= 16 &&
         W::lds_bytes(p.nasm) <= 160 * 1024) {
-      hipLaunchKernelGGL((k_asm_x_wide<N, HALVES>), dim3(ceil_div(nrows, W::rows())), dim3(64 * W::waves(p.nasm)),
+      hipLaunchKernelGGL((k_asm_x_wide<N, HALVES, PAD>), dim3(ceil_div(nrows, W::rows())), dim3(64 * W::waves(p.nasm)),
                          W::lds_bytes(p.nasm), s, p, tw);
       SIMR_LAUNCH_CHECK();
       return;
     }
   }
-  const bool lut = p.zdim >= 4 && p.nasm > 1 &&
-                   (long long)(p.nasm - 1) * p.ydim * N <= (long long)p.nasm * p.zdim * p.ny * p.nx;
   // small stacks: smaller workgroups, so that the rows spread over the CUs
-  int threads = C::MAXT;
-  while (threads > C::MINT && nrows < 1024LL * C::rows(threads)) threads /= 2;
-  const dim3 grid(ceil_div(nrows, C::rows(threads)));
-  const size_t lds = C::lds_bytes(threads, lut);
-  if (lut) {
-    hipLaunchKernelGGL(k_asm_phasors, dim3(ceil_div(N, 256), p.ydim, p.nasm - 1), dim3(256), 0, s, p,
-                       C::K::SPLIT ? 1 : 0, p.stageZ);
-    SIMR_LAUNCH_CHECK();
-    hipLaunchKernelGGL((k_asm_x<N, HALVES, true>), grid, dim3(threads), lds, s, p, tw, p.stageZ);
-  } else {
-    hipLaunchKernelGGL((k_asm_x<N, HALVES, false>), grid, dim3(threads), lds, s, p, tw, (const float2*)nullptr);
+  const auto threads_for = [](long long rows) {
+    int t = C::MAXT;
+    while (t > C::MINT && rows < 1024LL * C::rows(t)) t /= 2;
+    return t;
+  };
+  // the output rows whose phasors the table's place holds at a time
+  const long long per_row = (long long)(p.nasm - 1) * N, room = (long long)p.nasm * p.zdim * p.ny * p.nx;
+  const int parts = p.zdim >= 4 && p.nasm > 1 && per_row <= room ? ceil_div(p.ydim, room / per_row) : 0;
+  const int step = parts > 0 ? ceil_div(p.ydim, parts) : 0;
+  if (parts == 1 || (long long)step * p.zdim >= kAsmPartGroups * C::rows(C::MINT)) {
+    for (int y0 = 0; y0 < p.ydim; y0 += step) {
+      const int ny = p.ydim - y0 < step ? p.ydim - y0 : step;
+      const int threads = threads_for((long long)ny * p.zdim);
+      hipLaunchKernelGGL(k_asm_phasors, dim3(ceil_div(N, 256), ny, p.nasm - 1), dim3(256), 0, s, p,
+                         C::K::SPLIT ? 1 : 0, y0, p.stageZ);
+      SIMR_LAUNCH_CHECK();
+      hipLaunchKernelGGL((k_asm_x<N, HALVES, PAD, true>), dim3(ceil_div((long long)ny * p.zdim, C::rows(threads))),
+                         dim3(threads), C::lds_bytes(threads, true), s, p, y0, ny, tw, p.stageZ);
+      SIMR_LAUNCH_CHECK();
+    }
+    return;
   }
+  const int threads = threads_for(nrows);
+  hipLaunchKernelGGL((k_asm_x<N, HALVES, PAD, false>), dim3(ceil_div(nrows, C::rows(threads))), dim3(threads),
+                     C::lds_bytes(threads, false), s, p, 0, p.ydim, tw, (const float2*)nullptr);
   SIMR_LAUNCH_CHECK();
 }
 
@@ -299,9 +338,11 @@ static void asm_x_dispatch(const AsmParams& p, bool run, hipStream_t s) {
 #define SIMR_CASE(N)                            \
   case N:                                       \
     if (2 * p.nx == N)                          \
-      launch_asm_x_n<N, 2>(p, run, s);          \
+      launch_asm_x_n<N, 2, false>(p, run, s);   \
+    else if (2 * p.nx < N && rp_halves_pay<N>()) \
+      launch_asm_x_n<N, 2, rp_halves_pay<N>()>(p, run, s); \
     else                                        \
-      launch_asm_x_n<N, 1>(p, run, s);          \
+      launch_asm_x_n<N, 1, false>(p, run, s);   \
     return;
     SIMR_ZOOM_SIZES(SIMR_CASE)
 #undef SIMR_CASE

@@ -83,7 +83,24 @@ def assembled(p, bands, fits):
     return out
 
 
-@pytest.mark.parametrize("nx,ny,nz,phases,kw", CASES)
+# zooms above two and the two forms of the phasors: the halves of a length with empty
+# frequencies (1000, 1152, 1280, 2048, 2400 points; an odd height), whole lengths beside
+# them (3072, 4096), the table over the output rows in parts (the last one shorter),
+# phasors in the kernel with and without a remainder of their group
+ZOOMS = [
+    (80, 75, 4, 5, dict(zoomfact=16.0)),
+    (200, 240, 1, 3, dict(zoomfact=5.0)),
+    (360, 400, 3, 5, dict(zoomfact=3.2, bDampenOrder0=0)),
+    (512, 48, 5, 5, dict(zoomfact=4.0)),
+    (256, 300, 3, 5, dict(zoomfact=8.0, bDampenOrder0=0)),
+    (384, 96, 5, 5, dict(zoomfact=8.0)),
+    (400, 512, 6, 5, dict(zoomfact=4.0)),
+    (512, 16, 1, 3, dict(zoomfact=8.0)),
+    (240, 320, 8, 5, dict(zoomfact=4.0)),
+]
+
+
+@pytest.mark.parametrize("nx,ny,nz,phases,kw", CASES + ZOOMS)
 def test_assembly_sizes(nx, ny, nz, phases, kw):
     print("case %dx%dx%d, %d phases, %s" % (nx, ny, nz, phases, kw), flush=True)
     p, otf, raw, _ = synthetic(nx, ny, nz, nphases=phases, seed=nx + ny, gpu=True, **kw)

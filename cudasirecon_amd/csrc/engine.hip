@@ -228,7 +228,7 @@ Engine::Engine(const simr_params& p, const float* otf, int device) : P(p), L(Lay
   if (const char* e = std::getenv("SIMR_OVERLAPS_3PASS")) fused_ov_ = !(e[0] == '1' && e[1] == 0);
   // every twiddle table this context's transforms use (rows, columns, z, the
   // zoomed assembly lengths), so that no launch path allocates one
-  for (int n : {L.nx, L.ny, L.nz, L.xdim, L.ydim, L.zdim})
+  for (int n : {L.nx, L.nz, L.zdim})
     if (n > 1) (void)twiddles(n);
   for (int n : {L.ny, L.nz}) fft_cols_request_table(n);
   overlaps_request_tables(L.nx, L.ny);

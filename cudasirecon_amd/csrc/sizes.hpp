@@ -26,13 +26,18 @@
 
 // Axial lengths of the transforms in one thread's registers: 2 to 64 with
 // prime factors up to 31.  SIMR_REG_ONLY_SIZES: those that are not among
-// SIMR_Z_SIZES; SIMR_REG_SMALL_SIZES: all of them up to 32.
+// SIMR_Z_SIZES; SIMR_REG_SMALL_SIZES: all of them up to 32;
+// SIMR_REG_PAIR_SIZES: those of which two transforms fit a thread and that the
+// unpadded assembly takes (up to 21, and the ones up to 32 among REG_ONLY).
 #define SIMR_REG_ONLY_SIZES(X)                                                                    \
   X(11) X(13) X(17) X(19) X(22) X(23) X(26) X(29) X(31) X(33) X(34) X(38) X(39) X(44) X(46) X(51) \
   X(52) X(55) X(57) X(58) X(62)
 #define SIMR_REG_SMALL_SIZES(X)                                                                   \
   X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18)   \
   X(19) X(20) X(21) X(22) X(23) X(24) X(25) X(26) X(27) X(28) X(29) X(30) X(31) X(32)
+#define SIMR_REG_PAIR_SIZES(X)                                                                    \
+  X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18)   \
+  X(19) X(20) X(21) X(22) X(23) X(26) X(29) X(31)
 #define SIMR_REG_SIZES(X)                                                                         \
   SIMR_REG_SMALL_SIZES(X)                                                                         \
   X(33) X(34) X(35) X(36) X(38) X(39) X(40) X(42) X(44) X(45) X(46) X(48) X(49) X(50) X(51) X(52) \

@@ -367,6 +367,8 @@ __device__ __forceinline__ bool asm_dead(const AsmParams& p, int x, int y, float
   const float kx = (float)x * p.dkx, ky = (float)(2 * y > p.ny ? y - p.ny : y) * p.dky;
   return rc2 > 0.f && kx * kx + ky * ky > rc2;
 }
+// Unpadded depths up to here take their z pass in registers.
+constexpr int kAsmZRegMax = 21;
 bool asm_z_in_registers(const AsmParams& p);
 void launch_asm_z_reg(const AsmParams& p, hipStream_t s);
 // Requests the twiddle tables of the y and x passes (nx, ny, xdim, ydim are

@@ -164,7 +164,7 @@ constexpr int asm_zp_w() {
 }
 template <int N>
 constexpr bool asm_zp_ok() {
-  return N > 1 && 4 * fft_tpt(N) <= 256;
+  return N > kAsmZRegMax && 4 * fft_tpt(N) <= 256;
 }
 
 template <int N, bool B0>

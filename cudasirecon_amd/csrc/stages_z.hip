@@ -193,7 +193,7 @@ bool asm_z_in_registers(const AsmParams& p) {
 #undef SIMR_CASE
     only = true;
   }
-  return only || (p.zdim == p.nz && p.zdim <= 21);
+  return only || (p.zdim == p.nz && p.zdim <= kAsmZRegMax);
 }
 
 void launch_asm_z_reg(const AsmParams& p, hipStream_t s) {
@@ -205,7 +205,7 @@ void launch_asm_z_reg(const AsmParams& p, hipStream_t s) {
     hipLaunchKernelGGL((k_asm_z_reg<N, false>), grid, dim3(256), 0, s, p);   \
     SIMR_LAUNCH_CHECK();                                                     \
     return;
-      SIMR_REG_SMALL_SIZES(SIMR_CASE)
+      SIMR_REG_PAIR_SIZES(SIMR_CASE)
 #undef SIMR_CASE
     }
   }

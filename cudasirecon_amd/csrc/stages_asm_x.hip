@@ -20,16 +20,19 @@ namespace simr {
 //
 // What bounds it: the loads of the next band (three wavefronts per SIMD, 168
 // VGPRs) over vector arithmetic; with every input in cache 512 x 512 x 48
-// takes 362 us of the 518.  Prefetching a band ahead spills at 168 VGPRs (a
-// spilled register costs more than the wait), and at two wavefronts per SIMD
-// it gains 5% at 1024 columns and loses as much at 2048.  Planes slowest
+// takes 362 us of the 518.  Prefetching a band ahead spills at 168 VGPRs (and
+// then costs more than the wait), and at two wavefronts per SIMD
+// it gains 5% at 1024 columns and loses as much at 2048.  Lengths whose plans
+// have factors of 5 at 30 to 32 values a lane (200, 400, 480, 720, 800, 1440)
+// spill 25 to 42 registers at three wavefronts as it is, the others up to 5.  Planes slowest
 // instead of fastest: 575 us (the phasor table then misses the L2).  The
 // earlier form, eight bands side by side in a workgroup with the sum through
 // LDS, on zero-padded rows (radix-stage core where N = N1 N2, N1 | N2 had no
 // solution), against this one, per launch:
 //   1024 columns x 1024 x 48 planes  614 -> 518 us   768 x 768 x 26  639 -> 220 us
 //   2048 x 2048 x 16                2395 -> 743 us   960 x 800 x 21  745 -> 198 us
-//    512 x 512 x 32                  170 -> 107 us
+//    512 x 512 x 32                  170 -> 107 us   400 x 400 x 32  395 -> 118 us
+//    800 x 800 x 26                  894 -> 409 us   480 x 480 x 32  455 -> 153 us
 
 // modulation phasor of assembly band a (>= 1) at output column X of row Y
 // (cos_sin_kernel, gpuFunctionsImpl.cu:1942-1954: float angle, then sin/cos):
@@ -121,10 +124,11 @@ __device__ __forceinline__ void asm_x_fetch(const AsmParams& p, const float2* sr
   }
 }
 
-// Output rows y0 .. y0 + ny - 1 of every plane.
+// The first ny output rows of every plane at p.stageY and p.out (their planes
+// p.ydim rows apart); without the table, all of them.
 template <int N, int HALVES, bool PAD, bool LUT>
 __global__ __launch_bounds__((AsmX<N, HALVES>::MAXT), (AsmX<N, HALVES>::waves(LUT))) void k_asm_x(
-    AsmParams p, int y0, int ny, const float2* __restrict__ tw, const float2* __restrict__ lut) {
+    AsmParams p, int ny, const float2* __restrict__ tw, const float2* __restrict__ lut) {
 #pragma clang fp contract(off)
   using C = AsmX<N, HALVES>;
   using K = typename C::K;
@@ -143,15 +147,14 @@ __global__ __launch_bounds__((AsmX<N, HALVES>::MAXT), (AsmX<N, HALVES>::waves(LU
   const long long nrows = (long long)ny * p.zdim;
   const long long row = blk * (blockDim.x / T / (K::SPLIT ? 2 : 1)) + rslot;
   const long long rc = row < nrows ? row : nrows - 1;
-  const int yl = (int)(rc / p.zdim), z = (int)(rc - (long long)yl * p.zdim);
-  const int Y = y0 + yl;
+  const int Y = (int)(rc / p.zdim), z = (int)(rc - (long long)Y * p.zdim);
   const float2* src = p.stageY + ((long long)z * p.ydim + Y) * p.nx;
   const long long band = (long long)p.zdim * p.ydim * p.nx;
   const int jr = K::ROWS == T || j < K::ROWS ? j : K::ROWS - 1;
   const int X0 = K::out0(jr, odd ? 1 : 0);
   // the lane's phasors: entry pos0 + PSTEP k2 of each band's row
   constexpr int PSTEP = K::SPLIT ? N1 : K::ROWS;
-  const float2* ph = LUT ? lut + (long long)yl * N + (K::SPLIT && odd ? N / 2 : 0) + jr : nullptr;
+  const float2* ph = LUT ? lut + (long long)Y * N + (K::SPLIT && odd ? N / 2 : 0) + jr : nullptr;
   float2* phl = reinterpret_cast<float2*>(reinterpret_cast<float*>(twl + K::TABN) + blockDim.x / T * C::SPANP);
   float acc[N2];
 #pragma unroll 1
@@ -318,18 +321,21 @@ static void launch_asm_x_n(const AsmParams& p, bool run, hipStream_t s) {
     for (int y0 = 0; y0 < p.ydim; y0 += step) {
       const int ny = p.ydim - y0 < step ? p.ydim - y0 : step;
       const int threads = threads_for((long long)ny * p.zdim);
+      AsmParams q = p;
+      q.stageY += (long long)y0 * p.nx;
+      q.out += (long long)y0 * N;
       hipLaunchKernelGGL(k_asm_phasors, dim3(ceil_div(N, 256), ny, p.nasm - 1), dim3(256), 0, s, p,
                          C::K::SPLIT ? 1 : 0, y0, p.stageZ);
       SIMR_LAUNCH_CHECK();
       hipLaunchKernelGGL((k_asm_x<N, HALVES, PAD, true>), dim3(ceil_div((long long)ny * p.zdim, C::rows(threads))),
-                         dim3(threads), C::lds_bytes(threads, true), s, p, y0, ny, tw, p.stageZ);
+                         dim3(threads), C::lds_bytes(threads, true), s, q, ny, tw, p.stageZ);
       SIMR_LAUNCH_CHECK();
     }
     return;
   }
   const int threads = threads_for(nrows);
   hipLaunchKernelGGL((k_asm_x<N, HALVES, PAD, false>), dim3(ceil_div(nrows, C::rows(threads))), dim3(threads),
-                     C::lds_bytes(threads, false), s, p, 0, p.ydim, tw, (const float2*)nullptr);
+                     C::lds_bytes(threads, false), s, p, p.ydim, tw, (const float2*)nullptr);
   SIMR_LAUNCH_CHECK();
 }
 

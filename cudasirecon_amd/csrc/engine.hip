@@ -817,7 +817,7 @@ ModampSlots Engine::modamp_slots() const {
 // vector) at entries [at, at + n) of the zero-copy region: the candidates
 // travel in the kernel arguments, and the partials are summed per candidate on
 // the device (FP32 fit: in block order as cpuReduce, gpuFunctionsImpl_hh.cu:162-180;
-// FP64: in wave_sum's order), straight into the region.  The sums are
+// FP64: in quad_sum's), straight into the region.  The sums are
 // read (eval_read) after the next wait_fit().
 void Engine::eval_enqueue(const Cand* c, int n, int at) {
   SIMR_REQUIRE(n >= 1 && n <= kMaxCand && at >= 0 && at + n <= kZcCand, "modamp batch out of range");

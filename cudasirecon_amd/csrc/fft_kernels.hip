@@ -274,9 +274,10 @@ __global__ __launch_bounds__(W* fft2_tpt(N)) void k_fft2_rows(float2* __restrict
 // column, W adjacent columns (whole 128-byte lines) to a workgroup.  Bound by
 // HBM; the radix stages below keep the whole tile in LDS and pass through it
 // once a stage, which leaves fewer loads in flight (a quarter to a half of the
-// wavefronts at these lengths).  Forward y transform per launch, before and now:
-// 480x400x21 67.9 and 55.9 us, 384x384x26 64.3 and 61.5 (0.23 GB each way: 90 at
-// the rate of a copy for both launches, now 123), 480x360 9.7 and 7.0.  Longer
+// wavefronts at these lengths).  Forward y transform of a stack's bands, before
+// (every column) and now (the live ones): 480x400x21 137 us (241 columns) and 105
+// (224), 384x384x26 133 (193) and 116 (176: 0.42 GB, 3.6 TB/s), 480x360 10.3 and
+// 7.1; of the three correlations 9.8 and 7.4, 8.4 and 6.7, 9.1 and 6.1.  Longer
 // columns would hold more values a lane than three wavefronts leave room for.
 // A caller's own table (fft_cols' tw) has the radix stages' layout and stays there.
 template <int N>

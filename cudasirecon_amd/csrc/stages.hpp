@@ -178,8 +178,8 @@ void launch_modamp_fp32(const ModampSlots& m, const CandSet& c, int ncand, int n
                         float4* partials, hipStream_t s);
 // The sums of the modamp partials (the reference's host sum, cpuReduce,
 // gpuFunctionsImpl_hh.cu:162-180), on the device: for candidate c, its
-// partials (fp64: as wave_sum; fp32: in block order) and, fp64, its slot's
-// z-sum totals; out[4c..4c+3] = (xr, xi, sx, sy) (fp32: the float sums).  host_out: out is
+// partials (fp64: as quad_sum; fp32: in block order) and, fp64, its slot's
+// z-sum totals (as wave_sum); out[4c..4c+3] = (xr, xi, sx, sy) (fp32: the float sums).  host_out: out is
 // host memory, and the writes are made visible system-wide before the kernel
 // ends.
 void launch_modamp_evals(bool fp32, const ModampSlots& m, const CandSet& c, int ncand, const double2* part64,

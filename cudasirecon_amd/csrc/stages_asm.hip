@@ -312,6 +312,9 @@ struct AsmY {
   // wavefronts per SIMD asked of the register allocator (128 VGPRs each at
   // four, 168 at three): four where that does not spill.  Split halves and
   // factors of 5 do (800 rows: 29 registers, 243 us against 142 us at three).
+  // A workgroup of 512 threads is two wavefronts per SIMD whatever is asked for:
+  // 2304 and 4096 rows spill about 40 registers there (4096 x 2048 columns x 6
+  // planes 2.55 ms, on the radix stages before 2.33, the one length that lost).
   static constexpr int WAVES = VALUES <= 32 ? (K::SPLIT || LEN % 5 == 0 ? 3 : 4) : VALUES <= 40 ? 2 : 1;
   static constexpr int NT = W * GROUPS;
   static constexpr int LDS = lds_of(W);

@@ -407,6 +407,9 @@ __device__ __forceinline__ bool ov_col_live(const OvSupport& p, float2 range, in
 // a 512x512x48 stack (a launch is three directions), 350 in 1024x1024x16,
 // 29.0 in 256x256x32 and 11.2 in one 256x256 plane; now 149, 206, 26.0 and 12.6
 // (that one is latency: the shift, the profile, the bands, the twiddles).
+// A full OTF (RA = false) is looked up in eight places an element, and the longer
+// lengths' kernels keep part of their inputs in scratch (200 to 300 bytes a lane
+// at 480, 512 and 1024 rows, none at 64 and 256).
 // 480x400x21 and 384x384x26, at three passes before: the row pass's figures.
 template <int NY>
 constexpr int ovc_want() {
@@ -993,11 +996,11 @@ void launch_findpeak(int n, float2* cc, float* partial_val, int* partial_idx, fl
 // e^{i 2 pi dxy kx r}, x = 16 q + r, so a workgroup's few hundred sincos
 // (double, some 200 instructions) run once, side by side.
 // What bounds it: the latency of that chain at small sizes, the reads of P
-// (from the L2, 16 bytes a point for every group) at large ones.  A round of
-// 39 candidates: 256^2 7.2 -> 6.0 us, 512^2 13.7 -> 9.4, 1024^2 38 -> 19.4
-// against a candidate and four rows per workgroup with a sincos per column;
-// 16 rows 14.6 and 30.1 us at the two larger sizes (too few workgroups); groups of
-// two the same.
+// (from the L2, 16 bytes a point for every group) at large ones.  A round of 13
+// candidates (of at most kFitReq) for each of three directions: 256^2 7.2 -> 6.0
+// us, 512^2 13.7 -> 9.4, 1024^2 38 -> 19.4 against a candidate and four rows per
+// workgroup with a sincos per column; 16 rows 14.6 and 30.1 us at the two larger
+// sizes (too few workgroups); groups of two the same.
 constexpr int kModGroup = 4;
 constexpr int kModRows = 8;
 int modamp_partials_fp64(int nx, int ny) { return (ny + kModRows - 1) / kModRows; }
